@@ -92,6 +92,39 @@ def test_act_quant_group128_bit_exact(ctx, oracle):
         assert np.array_equal(host(q), qo) and np.array_equal(host(s), so), group
 
 
+@pytest.mark.parametrize("rows,k", [(1, 128), (3, 384), (7, 1152)])
+def test_act_quant_alignment_and_odd_sizes(ctx, oracle, rows, k):
+    """The float4 kernel (shift 0) and the one-thread-per-group kernel that
+    takes an x or q off its alignment, at sizes that leave a workgroup partly
+    filled: both equal the oracle, and each other where a group holds an
+    infinity (whose scale the oracle does not define)."""
+    say(f"act quant rows={rows} k={k}")
+    rng = np.random.default_rng(rows * k)
+    x = (rng.standard_normal((rows, k)) * np.exp(rng.uniform(-6, 6, (rows, k)))).astype(np.float32)
+    x[0, 3], x[-1, -1], x[0, 64] = 1e30, -np.nan, 0.0
+    xi = x.copy()
+    xi[0, 5], xi[-1, k // 2] = np.inf, -np.inf
+
+    def quant(v, shift, group):
+        flat = torch.zeros(rows * k + 4, dtype=torch.float32, device="cuda")
+        xd = flat[shift:shift + rows * k].view(rows, k)
+        xd.copy_(dev(v))
+        qf = torch.zeros(rows * k + 4, dtype=torch.uint8, device="cuda")
+        q = qf[shift:shift + rows * k].view(rows, k)
+        s = torch.empty((rows, k // group), dtype=torch.uint8, device="cuda")
+        s14.act_quant_e4m3(ctx, xd, q, s, group=group)
+        assert not host(qf)[shift + rows * k:].any() and not host(qf)[:shift].any()
+        return host(q), host(s)
+
+    for group in (128, 64, 32):
+        want = oracle.requant_e4m3(x, group=group)
+        for shift in (0, 1, 2):
+            got = quant(x, shift, group)
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), (group, shift)
+        a, b = quant(xi, 0, group), quant(xi, 1, group)
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]), group
+
+
 @pytest.mark.parametrize("m", [1, 4])
 @pytest.mark.parametrize("name", list(SHAPES))
 def test_fp8_linear_projection_shapes(ctx, oracle, name, m):
