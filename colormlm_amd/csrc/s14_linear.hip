@@ -38,7 +38,9 @@
 namespace s14 {
 namespace {
 
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 // Eight e4m3 codes (two little-endian words) as eight bf16, exactly.
@@ -181,7 +183,8 @@ __global__ __launch_bounds__(256) void k_linear_exact(LinearArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// EXACT, tiled (k % 128 == 0, 16-byte aligned x and w): one wavefront per
+// EXACT, tiled (k % 128 == 0, 16-byte aligned x and w; f32 scales, whose
+// products are not exact in f32, or few tokens over a long k): one wavefront per
 // (64-row tile, scale group g, block of MT tokens), four independent
 // wavefronts per workgroup.  The wavefront DMA-loads its 64 rows x 128 bytes
 // of weight into LDS (buffer_load ... lds: 8 lanes per row, whole lines per
@@ -850,6 +853,241 @@ __global__ __launch_bounds__(64 * kGxWaves) void k_linear_gemv_exact(LinearArgs 
   a.y[r0 + lane] = v;
 }
 
+// ---------------------------------------------------------------------------
+// EXACT on the f32 matrix cores (k % 128 == 0, UE8M0 scales on both sides).
+// An e4m3 x e4m3 product has at most eight significant bits, so in f32 it is
+// exact and the oracle's multiply-then-add equals one fused multiply-add; the
+// one-k f32 MFMAs are exactly that, one rounding per k with k ascending (the
+// rounding checked against fmaf chains, subnormals included).  The scales
+// are powers of two: with every code of a group in the window below, the sum
+// of the raw codes' products times 2^(cx + cw - 254) is the oracle's partial
+// bit for bit.  A multiply and an add per product on the vector units
+// (k_linear_tile) issue 8 products a cycle and SIMD, these MFMAs 32.
+//
+// A workgroup owns 64 rows x kT kNB tokens; its W wavefronts take the groups
+// in turn (wavefront w: W r + w) and leave their partials in LDS, where the
+// row's owner adds them in group order (acc = 0; acc += partial_g).  No
+// partial goes to memory.  A group's weights (8 KiB) and its tokens' codes
+// come by coalesced DMA loads into LDS, from where the lane that feeds a row
+// takes its 128 bytes to registers; the next group's loads are in flight
+// during the products.  (Loaded straight to registers, 64 rows' 16 bytes an
+// instruction, the loads' addresses bound the kernel.)  Lane l feeds row l
+// and token l % kT; a lane's result quads: kT = 32 (v_mfma_f32_32x32x1_2b)
+// rows 8 q + 4 (l / 32) + j, kT = 16 (16x16x1_4b) rows 16 q + 4 (l / 16) + j,
+// kT = 4 (4x4x1_16b) rows 4 (l / 4) + j.
+// Bound by the MFMAs and the code conversions, which on these units add up
+// (a timed loop of one f32 MFMA and one conversion takes the sum of the two):
+// 64 rows x 32 tokens x 128 k take 3.84 us of MFMA, 4.7 us here.
+// ---------------------------------------------------------------------------
+template <int kT>
+struct XmAcc;
+template <>
+struct XmAcc<16> {
+  typedef v16f type;
+  static __device__ __forceinline__ type mfma(float a, float b, type c) {
+    return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct XmAcc<32> {
+  typedef v32f type;
+  static __device__ __forceinline__ type mfma(float a, float b, type c) {
+    return __builtin_amdgcn_mfma_f32_32x32x1f32(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct XmAcc<4> {
+  typedef v4f type;
+  static __device__ __forceinline__ type mfma(float a, float b, type c) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
+  }
+};
+constexpr uint32_t kXmRows = 64;
+
+// Four e4m3 codes as f32, exactly.
+__device__ __forceinline__ void e4m3x4_f32(float (&v)[4], uint32_t w) {
+  const v2f lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w, 1.0f, false);
+  const v2f hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w, 1.0f, true);
+  v[0] = lo.x, v[1] = lo.y, v[2] = hi.x, v[3] = hi.y;
+}
+
+template <int kT, int kNB, int W>
+__global__ __launch_bounds__(64 * W) void k_linear_exact_mfma(LinearArgs a, uint32_t tok_blocks, uint32_t total) {
+  typedef typename XmAcc<kT>::type Acc;
+  constexpr uint32_t kQ = kT / 4, kQuads = kQ * uint32_t(kNB);  // result quads per token block, and in all
+  constexpr uint32_t kTok = uint32_t(kT * kNB);
+  __shared__ __attribute__((aligned(16))) float4 xm_part[W][kQuads][64];
+  __shared__ __attribute__((aligned(16))) uint8_t xm_w[W][kXmRows * kLinGroup];
+  __shared__ __attribute__((aligned(16))) uint8_t xm_x[W][kTok * kLinGroup];
+  // workgroup p of a contiguous run per XCD (workgroups go to the 8 XCDs in
+  // turn): the token blocks of one row tile share its weights in one L2
+  const uint32_t per = gridDim.x / 8u;
+  const uint32_t p = (blockIdx.x % 8u) * per + blockIdx.x / 8u;
+  if (p >= total) return;  // the whole workgroup
+  const uint32_t tile = p / tok_blocks, m0 = (p % tok_blocks) * kTok, r0 = tile * kXmRows;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  const uint32_t G = a.groups, K = a.k, N = a.n, M = a.m;
+  const Rsrc rw = make_rsrc(a.w, N * K), rx = make_rsrc(a.x, M * K);
+  const Rsrc rsw = make_rsrc(a.w_scale, (N + 127u) / 128u * G), rsx = make_rsrc(a.x_scale, M * G);
+  // DMA lane map: load j of a group's weights moves rows 8 j .. 8 j + 7, lane
+  // l the piece (l % 8) ^ (row & 7) of row 8 j + l / 8 (landing at piece
+  // l % 8); the same for the tokens' codes.  Rows past n read zeros; tokens
+  // past m take the last one's codes and are not stored.
+  const uint32_t drow = lane >> 3, dpiece = 16u * ((lane & 7u) ^ drow);
+  uint32_t cw, cx[kNB];
+  auto issue = [&](uint32_t g) {
+#pragma unroll
+    for (uint32_t j = 0; j < kXmRows / 8u; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lt_lds_void *)(xm_w[wave] + 1024u * j), 16,
+                                               (r0 + 8u * j + drow) * K + g * kLinGroup + dpiece, 0, 0, 0);
+    if constexpr (kTok >= 8u) {
+#pragma unroll
+      for (uint32_t j = 0; j < kTok / 8u; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lt_lds_void *)(xm_x[wave] + 1024u * j), 16,
+                                                 min(m0 + 8u * j + drow, M - 1u) * K + g * kLinGroup + dpiece, 0, 0, 0);
+    } else {  // four tokens: the lanes past them repeat the last one's line into an unused part
+      if (lane < 8u * kTok)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lt_lds_void *)(xm_x[wave]), 16,
+                                                 min(m0 + drow, M - 1u) * K + g * kLinGroup + dpiece, 0, 0, 0);
+    }
+    cw = ld1(rsw, (r0 / 128u) * G + g);
+#pragma unroll
+    for (int b = 0; b < kNB; ++b) cx[b] = ld1(rsx, min(m0 + uint32_t(kT * b) + lane % kT, M - 1u) * G + g);
+  };
+  if (wave < G) issue(wave);
+  uint4 A[8], B[kNB][8];
+  constexpr uint32_t kOwn = (kQuads + W - 1) / W;  // quads a wavefront folds: wave, wave + W, ..
+  float4 tot[kOwn];
+#pragma unroll
+  for (uint32_t o = 0; o < kOwn; ++o) tot[o] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 1
+  for (uint32_t g0 = 0; g0 < G; g0 += W) {
+    const uint32_t g = g0 + wave;
+    if (g < G) {
+      // this group's codes out of LDS, then the next group's on their way
+      // into it during this one's products
+#pragma unroll
+      for (uint32_t c = 0; c < 8; ++c) {
+        A[c] = *reinterpret_cast<const uint4 *>(xm_w[wave] + kLinGroup * lane + 16u * (c ^ (lane & 7u)));
+#pragma unroll
+        for (int b = 0; b < kNB; ++b) {
+          const uint32_t t = uint32_t(kT * b) + lane % kT;
+          B[b][c] = *reinterpret_cast<const uint4 *>(xm_x[wave] + kLinGroup * t + 16u * (c ^ (t & 7u)));
+        }
+      }
+      bool in = true;
+      const uint32_t cwg = cw;
+      uint32_t cxg[kNB];
+#pragma unroll
+      for (int b = 0; b < kNB; ++b) cxg[b] = cx[b];
+      lin_lds_reads_done();
+      asm volatile("" ::: "memory");
+      if (g + W < G) issue(g + W);
+#pragma unroll
+      for (int b = 0; b < kNB; ++b)
+        in = in && cxg[b] >= 10u && cxg[b] <= 246u && cwg >= 10u && cwg <= 246u && cxg[b] + cwg >= 146u && cxg[b] + cwg <= 356u;
+      if (__all(in)) {
+        float s[kNB];
+#pragma unroll
+        for (int b = 0; b < kNB; ++b) s[b] = __uint_as_float((cxg[b] + cwg - 127u) << 23);
+        Acc acc[kNB];
+#pragma unroll
+        for (int b = 0; b < kNB; ++b) acc[b] = Acc{};
+#pragma unroll
+        for (uint32_t c = 0; c < 8; ++c) {
+          const uint32_t ww[4] = {A[c].x, A[c].y, A[c].z, A[c].w};
+          uint32_t xw[kNB][4];
+#pragma unroll
+          for (int b = 0; b < kNB; ++b) xw[b][0] = B[b][c].x, xw[b][1] = B[b][c].y, xw[b][2] = B[b][c].z, xw[b][3] = B[b][c].w;
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            float av[4], bv[kNB][4];
+            e4m3x4_f32(av, ww[d]);
+#pragma unroll
+            for (int b = 0; b < kNB; ++b) e4m3x4_f32(bv[b], xw[b][d]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+              for (int b = 0; b < kNB; ++b) acc[b] = XmAcc<kT>::mfma(av[i], bv[b][i], acc[b]);
+          }
+        }
+#pragma unroll
+        for (int b = 0; b < kNB; ++b)
+#pragma unroll
+          for (uint32_t q = 0; q < kQ; ++q)
+            xm_part[wave][uint32_t(b) * kQ + q][lane] =
+                make_float4(__fmul_rn(acc[b][4 * q], s[b]), __fmul_rn(acc[b][4 * q + 1], s[b]),
+                            __fmul_rn(acc[b][4 * q + 2], s[b]), __fmul_rn(acc[b][4 * q + 3], s[b]));
+      } else {
+        // a scale outside the window: the oracle's separate multiplies, lane
+        // = row, one token at a time (its codes read from the lane that holds them)
+        const float sb = ue8m0_f32(cwg);
+#pragma unroll
+        for (int b = 0; b < kNB; ++b) {
+#pragma unroll 1
+          for (uint32_t t = 0; t < uint32_t(kT); ++t) {
+            const float sa = ue8m0_f32(uint32_t(__builtin_amdgcn_readlane(int(cxg[b]), int(t))));
+            float sum = 0.0f;
+#pragma unroll
+            for (uint32_t c = 0; c < 8; ++c) {
+              const uint32_t ww[4] = {A[c].x, A[c].y, A[c].z, A[c].w};
+              const uint32_t xw[4] = {B[b][c].x, B[b][c].y, B[b][c].z, B[b][c].w};
+#pragma unroll
+              for (int d = 0; d < 4; ++d) {
+                float av[4], bv[4];
+                uint32_t w = ww[d];
+                asm volatile("" : "+v"(w));  // decoded anew per token: hoisted, the row would hold 128 registers
+                e4m3x4_f32(av, uint32_t(__builtin_amdgcn_readlane(int(xw[d]), int(t))));
+                e4m3x4_f32(bv, w);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                  sum = __fadd_rn(sum, __fmul_rn(__fmul_rn(av[i], sa), __fmul_rn(bv[i], sb)));
+              }
+            }
+            const uint32_t q = kT == 32 ? lane / 8u : kT == 16 ? lane / 16u : 0u;
+            const uint32_t dl = kT == 32   ? lane % 8u / 4u * 32u + t
+                                : kT == 16 ? lane % 16u / 4u * 16u + t
+                                           : lane / 4u * 4u + t;
+            reinterpret_cast<float *>(&xm_part[wave][uint32_t(b) * kQ + q][dl])[lane % 4u] = sum;
+          }
+        }
+      }
+    }
+    __syncthreads();
+    const uint32_t live = min(uint32_t(W), G - g0);
+#pragma unroll
+    for (uint32_t o = 0; o < kOwn; ++o) {
+      const uint32_t quad = wave + uint32_t(W) * o;
+      if (quad < kQuads)
+        for (uint32_t w = 0; w < live; ++w) {
+          const float4 v = xm_part[w][quad][lane];
+          tot[o] = make_float4(__fadd_rn(tot[o].x, v.x), __fadd_rn(tot[o].y, v.y), __fadd_rn(tot[o].z, v.z),
+                               __fadd_rn(tot[o].w, v.w));
+        }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (uint32_t o = 0; o < kOwn; ++o) {
+    const uint32_t quad = wave + uint32_t(W) * o;
+    if (quad >= kQuads) continue;
+    const uint32_t m = m0 + uint32_t(kT) * (quad / kQ) + lane % kT;
+    const uint32_t row = r0 + (kT == 32   ? 8u * (quad % kQ) + 4u * (lane / 32u)
+                               : kT == 16 ? 16u * (quad % kQ) + 4u * (lane / 16u)
+                                          : 4u * (lane / 4u));
+    if (m >= M) continue;
+    const float v[4] = {tot[o].x, tot[o].y, tot[o].z, tot[o].w};
+    float *y = a.y + size_t(m) * N + row;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      if (row + j >= N) break;
+      float f = v[j];
+      if (a.bias) f = __fadd_rn(f, a.bias[row + j]);
+      y[j] = a.round_bf16 ? bf16_round(f) : f;
+    }
+  }
+}
+
 }  // namespace
 
 hipError_t launch_act_quant(hipStream_t s, uint32_t rows, uint32_t k, uint32_t group, const float *x, uint8_t *q,
@@ -990,6 +1228,27 @@ static void launch_gemv_exact(hipStream_t s, const LinearArgs &a) {
     k_linear_gemv_exact<R, false, false><<<grid, 64 * kGxWaves, 0, s>>>(a);
 }
 
+template <int kT, int kNB, int W>
+static hipError_t launch_exact_mfma(hipStream_t s, const LinearArgs &a) {
+  const uint32_t tok_blocks = (a.m + kT * kNB - 1) / (kT * kNB);
+  const uint32_t total = (a.n + kXmRows - 1) / kXmRows * tok_blocks;
+  k_linear_exact_mfma<kT, kNB, W><<<(total + 7u) / 8u * 8u, 64 * W, 0, s>>>(a, tok_blocks, total);
+  return hipGetLastError();
+}
+
+static hipError_t launch_exact_plan(hipStream_t s, const LinearArgs &a, const LinExactPlan &p) {
+  switch (p.tokens * 100u + p.waves) {
+    case 404u: return launch_exact_mfma<4, 1, 4>(s, a);
+    case 416u: return launch_exact_mfma<4, 1, 16>(s, a);
+    case 804u: return launch_exact_mfma<4, 2, 4>(s, a);
+    case 808u: return launch_exact_mfma<4, 2, 8>(s, a);
+    case 1604u: return launch_exact_mfma<16, 1, 4>(s, a);
+    case 1608u: return launch_exact_mfma<16, 1, 8>(s, a);
+    case 3204u: return launch_exact_mfma<32, 1, 4>(s, a);
+    default: return hipErrorInvalidValue;  // no such plan
+  }
+}
+
 hipError_t launch_fp8_linear(hipStream_t s, const LinearArgs &a, int mode, const LinearWorkspace &ws) {
   // the GEMV where it measured faster than the MFMA tiles (graph replays,
   // us: wq_b m = 1 8.5 against 10.4, m = 2 10.9 against 10.7; wo_a m = 2 11.2
@@ -1040,6 +1299,12 @@ hipError_t launch_fp8_linear(hipStream_t s, const LinearArgs &a, int mode, const
     }
     return hipGetLastError();
   }
+  // the f32 MFMA: UE8M0 scales, whole groups.  Two to four tokens over a k
+  // past 4,096 stay on the tiles below (wo_b m = 4: 21.5 us against 24.1:
+  // 64-row workgroups leave most CUs idle there)
+  if (vec && a.k % kLinGroup == 0u && !a.x_scale_f32 && !a.w_scale_f32 && (a.m > 4u || a.k <= 4096u) &&
+      uint64_t(a.n + kXmRows - 1) * a.k <= 0xFFFFFFFFull)
+    return launch_exact_plan(s, a, lin_exact_plan(a.m, a.n, a.groups));
   // tiled: whole groups, one token's partials within the workspace, and the
   // last tile's row offsets within 32 bits (rows past n read zeros)
   if (vec && a.k % kLinGroup == 0u && size_t(a.groups) * a.n * sizeof(float) <= kLinPartBytes &&

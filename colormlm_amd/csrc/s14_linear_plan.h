@@ -70,4 +70,35 @@ inline LinFastPlan lin_fast_plan(uint32_t m, uint32_t n, uint32_t G) {
   }
 }
 
+// EXACT on the f32 MFMA (k_linear_exact_mfma): tokens per workgroup and
+// wavefronts per workgroup, the pair with the least estimated time.  A
+// workgroup is 64 rows x `tokens`; its wavefronts take ceil(G / waves) groups
+// each, and whole rounds of 256 workgroups count.  ns per group of four
+// wavefronts, measured at wo_a and wo_b with at most one workgroup per CU
+// (alone) and with several: few wide tiles leave MFMA latency and the LDS
+// reads uncovered, many small ones convert the same weights more often.
+struct LinExactPlan {
+  uint32_t tokens, waves;
+};
+inline LinExactPlan lin_exact_plan(uint32_t m, uint32_t n, uint32_t G) {
+  struct Kind {
+    uint32_t tokens, waves, alone_ns, shared_ns;
+  };
+  constexpr Kind kinds[] = {{4, 4, 1760, 1110},  {4, 16, 1220, 1420}, {8, 4, 3000, 1900},  {8, 8, 2400, 2500},
+                            {16, 4, 3200, 2600}, {16, 8, 2650, 2850}, {32, 4, 5300, 4660}};
+  const uint64_t tiles = (uint64_t(n) + 63u) / 64u;
+  LinExactPlan best{0, 0};
+  uint64_t least = ~uint64_t(0);
+  for (const Kind &k : kinds) {
+    const uint64_t wgs = tiles * ((uint64_t(m) + k.tokens - 1u) / k.tokens);
+    const uint64_t t = (wgs + 255u) / 256u * ((G + k.waves - 1u) / k.waves) * (k.waves / 4u) *
+                       (wgs <= 256u ? k.alone_ns : k.shared_ns);
+    if (t < least) {
+      least = t;
+      best = {k.tokens, k.waves};
+    }
+  }
+  return best;
+}
+
 }  // namespace s14

@@ -238,6 +238,36 @@ def test_fp8_linear_exact_one_token_extreme_scales(ctx, oracle, k):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.count_nonzero(got != want)
 
 
+@pytest.mark.parametrize("m,n,k", [(2, 300, 384), (3, 64, 128), (5, 4160, 1152), (7, 129, 4096), (13, 1000, 640),
+                                   (17, 8192, 256), (31, 2000, 1536), (33, 16450, 512), (65, 700, 2176),
+                                   (97, 8200, 384), (160, 12288, 256),
+                                   (52, 4160, 640), (132, 1000, 640), (12, 8192, 2048)])
+def test_fp8_linear_exact_mfma_plans(ctx, oracle, m, n, k):
+    """The f32-MFMA EXACT kernel with every plan (4, 8, 16 and 32 tokens per
+    workgroup; 4, 8 and 16 wavefronts): rows cut inside a 64-row tile,
+    tokens cut inside a block, fewer groups than wavefronts and a ragged last
+    round of groups; then UE8M0 codes that leave the MFMA's window (0..12, so
+    that products fall to subnormals or zero), a bias and bf16 outputs; bit
+    for bit."""
+    say(f"fp8_linear exact mfma m={m} n={n} k={k}")
+    rng = np.random.default_rng(m * n + k)
+    w, x = codes(rng, (n, k)), codes(rng, (m, k))
+    b = rng.standard_normal(n).astype(np.float32)
+    for extreme in (False, True):
+        ws = rng.integers(114, 122, (-(-n // 128), k // 128), dtype=np.uint8)
+        xs = rng.integers(118, 128, (m, k // 128), dtype=np.uint8)
+        if extreme:
+            for a in (ws, xs):
+                sel = rng.random(a.shape) < 0.2
+                a[sel] = rng.integers(0, 13, int(sel.sum()), dtype=np.uint8)
+        y = torch.full((m, n), np.nan, dtype=torch.float32, device="cuda")
+        kw = {"bias": dev(b), "round_bf16": True} if extreme else {}
+        s14.fp8_linear(ctx, dev(x), dev(xs), dev(w), dev(ws), y, mode=s14.EXACT, **kw)
+        want = oracle.fp8_linear(x, xs, w, ws, **({"bias": b, "round_bf16": True} if extreme else {}))
+        got = host(y)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (extreme, np.count_nonzero(got != want))
+
+
 def test_fp8_linear_exact_token_chunks(ctx, oracle):
     """EXACT keeps every group partial of a launch in the context's 32 MiB
     workspace: at wq_b's shape (8 groups x 32768 rows x 4 bytes per token)
