@@ -631,6 +631,169 @@ __global__ __launch_bounds__(64) void k_linear_fast(LinearArgs a, LinearWorkspac
   }
 }
 
+// ---------------------------------------------------------------------------
+// FAST for prompts: a workgroup owns 128 rows (one scale block) x 16 TT
+// tokens and a range of scale groups, wavefront w its rows 32 w .. 32 w + 31.
+// Per group of 128 k the tokens' codes are decoded to bf16 once for the
+// workgroup into one of two LDS buffers (with UE8M0 scales the power of two
+// sa[t][g] * sb[g] folded in exactly), while the weights, which only their
+// own wavefront reads, come straight to registers and are decoded there, one
+// group ahead.  v_mfma_f32_16x16x32_bf16, lane l = (c, q) = (l % 16, l / 16):
+// in MFMA j of a group it feeds row (token) c at k 32 q + 8 j .. + 7, so a
+// lane's weights are 32 contiguous bytes and its token operand one 16-byte
+// LDS read; result element v is row 4 q + v, token c.  Piece p of a token's
+// 256 bytes sits at p ^ (token & 15).  Sums of kLgFlush groups (one with f32
+// scales, scaled by sa * sb) are added to the running sums, which keeps the
+// rounding of the 512-k sums that k_linear_fast's splits make.  K splits
+// (of 512 k at least) leave their sums in the workspace for k_linear_sum.
+// Bound by the decoding, the MFMAs and the LDS reads in turn: 54 us for 512
+// tokens of wo_a, where the MFMAs alone take 20 (k_linear_fast, one wavefront
+// per 32 x 32 tile and split, 557).  Measured and not kept: 128 tokens a
+// workgroup (one workgroup per CU by registers: 58), every group's sums
+// joined on their own (85), scheduling groups that place the decoding between
+// the MFMAs by hand (61 to 68).
+// ---------------------------------------------------------------------------
+constexpr uint32_t kLgWaves = 4, kLgRows = 32u * kLgWaves;
+constexpr uint32_t kLgFlush = 4;
+template <int TT, bool kXsF32, bool kWsF32>
+__global__ __launch_bounds__(64 * kLgWaves) void k_linear_gemm(LinearArgs a, float *__restrict__ part, uint32_t tok_blocks,
+                                                     uint32_t total, uint32_t per_split) {
+  constexpr bool kFold = !kXsF32 && !kWsF32;
+  constexpr uint32_t kTok = 16u * uint32_t(TT), kLd = kTok * 8u / (64u * kLgWaves);  // tokens; 16-byte code loads per thread
+  __shared__ __attribute__((aligned(16))) uint8_t lg_x[2][kTok][2u * kLinGroup];
+  __shared__ float lg_s[2][kTok];
+  // token blocks of one row tile next to each other in a contiguous run per XCD
+  const uint32_t p = (blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
+  if (p >= total) return;  // the whole workgroup
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, c = lane & 15u, q = lane >> 4;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t K = a.k, N = a.n, M = a.m, G = a.groups;
+  const uint32_t m0 = (p % tok_blocks) * kTok, rest = p / tok_blocks;
+  const uint32_t tiles = (N + kLgRows - 1u) / kLgRows, tile = rest % tiles, split = rest / tiles;
+  const uint32_t g0 = split * per_split, g1 = min(g0 + per_split, G), r0 = tile * kLgRows + 32u * wave;
+  const Rsrc rw = make_rsrc(a.w, N * K), rx = make_rsrc(a.x, M * K);
+  const uint32_t n_sw = (N + 127u) / 128u * G, n_sx = M * G;
+  const Rsrc rsw = make_rsrc(a.w_scale, kWsF32 ? 4u * n_sw : n_sw);
+  const Rsrc rsx = make_rsrc(a.x_scale, kXsF32 ? 4u * n_sx : n_sx);
+  // rows past n read zeros; tokens past m take the last one's, not stored
+  const uint32_t woff = (r0 + c) * K + 32u * q;
+  uint32_t tok[kLd];
+#pragma unroll
+  for (uint32_t i = 0; i < kLd; ++i) tok[i] = min(m0 + (64u * kLgWaves * i + tid) / 8u, M - 1u);
+  const uint32_t piece = tid & 7u;
+  uint4 aw[2][2], xw[kLd];
+  float sw, sx[kLd];
+  auto load_w = [&](uint32_t g) {
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i)
+#pragma unroll
+      for (uint32_t h = 0; h < 2; ++h) aw[i][h] = ld16(rw, woff + 16u * i * K + g * kLinGroup + 16u * h);
+  };
+  auto load_x = [&](uint32_t g) {
+    sw = lin_scale(rsw, tile * G + g, kWsF32);
+#pragma unroll
+    for (uint32_t i = 0; i < kLd; ++i) {
+      xw[i] = ld16(rx, tok[i] * K + g * kLinGroup + 16u * piece);
+      sx[i] = lin_scale(rsx, tok[i] * G + g, kXsF32);
+    }
+  };
+  auto store_x = [&](uint32_t b) {
+#pragma unroll
+    for (uint32_t i = 0; i < kLd; ++i) {
+      const uint32_t t = (64u * kLgWaves * i + tid) / 8u;
+      const float s = sx[i] * sw, f = kFold ? s : 1.0f;
+      *reinterpret_cast<v4u *>(&lg_x[b][t][16u * ((2u * piece) ^ (t & 15u))]) = e4m3x4_bf16s(xw[i].x, xw[i].y, f);
+      *reinterpret_cast<v4u *>(&lg_x[b][t][16u * ((2u * piece + 1u) ^ (t & 15u))]) = e4m3x4_bf16s(xw[i].z, xw[i].w, f);
+      if constexpr (!kFold)
+        if (piece == 0) lg_s[b][t] = s;
+    }
+  };
+  v8bf av[2][2][4];  // decoded weights of this group and the next, in turn
+  auto cvt_w = [&](v8bf (&d)[2][4], uint32_t i) {
+    d[i][0] = e4m3x8_bf16(aw[i][0].x, aw[i][0].y), d[i][1] = e4m3x8_bf16(aw[i][0].z, aw[i][0].w);
+    d[i][2] = e4m3x8_bf16(aw[i][1].x, aw[i][1].y), d[i][3] = e4m3x8_bf16(aw[i][1].z, aw[i][1].w);
+  };
+  load_x(g0);
+  load_w(g0);
+  store_x(0);
+  cvt_w(av[0], 0);
+  cvt_w(av[0], 1);
+  load_x(min(g0 + 1u, g1 - 1u));
+  load_w(min(g0 + 1u, g1 - 1u));
+  v4f acc[2][TT], sum[2][TT];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int t = 0; t < TT; ++t) acc[i][t] = v4f{}, sum[i][t] = v4f{};
+  __syncthreads();
+  // group g from buffer b: its MFMAs, with the next group's decoding between them
+  auto step = [&](auto tag, uint32_t g) {
+    constexpr uint32_t b = decltype(tag)::value;
+    store_x(b ^ 1u);
+    cvt_w(av[b ^ 1u], 0);
+    cvt_w(av[b ^ 1u], 1);
+    load_w(min(g + 2u, g1 - 1u));
+    load_x(min(g + 2u, g1 - 1u));
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) {
+        const v8bf xv = *reinterpret_cast<const v8bf *>(&lg_x[b][16u * uint32_t(t) + c][16u * ((4u * q + j) ^ c)]);
+        acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[b][0][j], xv, acc[0][t], 0, 0, 0);
+        acc[1][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[b][1][j], xv, acc[1][t], 0, 0, 0);
+      }
+    }
+    if (!kFold || (g - g0) % kLgFlush == kLgFlush - 1u || g + 1u == g1) {
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        const float s = kFold ? 1.0f : lg_s[b][16u * uint32_t(t) + c];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) sum[i][t][v] = kFold ? sum[i][t][v] + acc[i][t][v] : fmaf(acc[i][t][v], s, sum[i][t][v]);
+          acc[i][t] = v4f{};
+        }
+      }
+    }
+    __syncthreads();
+  };
+  uint32_t g = g0;
+#pragma unroll 1
+  for (; g + 1u < g1; g += 2u) {
+    step(std::integral_constant<uint32_t, 0>{}, g);
+    step(std::integral_constant<uint32_t, 1>{}, g + 1u);
+  }
+  if (g < g1) step(std::integral_constant<uint32_t, 0>{}, g);
+  float *out = part ? part + size_t(split) * M * N : a.y;
+  const bool vec = N % 4u == 0u && (reinterpret_cast<uintptr_t>(out) & 15u) == 0u;
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    const uint32_t m = m0 + 16u * uint32_t(t) + c;
+    if (m >= M) continue;
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+      const uint32_t row = r0 + 16u * i + 4u * q;
+      if (row >= N) continue;
+      float o[4] = {sum[i][t][0], sum[i][t][1], sum[i][t][2], sum[i][t][3]};
+      if (!part) {
+#pragma unroll
+        for (uint32_t v = 0; v < 4; ++v) {
+          if (a.bias && row + v < N) o[v] += a.bias[row + v];
+          if (a.round_bf16) o[v] = bf16_round(o[v]);
+        }
+      }
+      float *dst = out + size_t(m) * N + row;
+      if (vec) {
+        *reinterpret_cast<float4 *>(dst) = make_float4(o[0], o[1], o[2], o[3]);
+      } else {
+#pragma unroll
+        for (uint32_t v = 0; v < 4; ++v)
+          if (row + v < N) dst[v] = o[v];
+      }
+    }
+  }
+}
+
 // FAST for one or two tokens (up to four where n is small) and k a multiple
 // of 1,024: a VALU GEMV,
 // where the MFMA path would spend 32-token tiles on one token.  One
@@ -1153,6 +1316,20 @@ static void launch_tile_mt(hipStream_t s, const LinearArgs &a, float *part) {
     k_linear_tile<MT, false, false><<<grid, 64 * kLTWaves, 0, s>>>(a, part);
 }
 
+// The K splits' sums (or the groups'), in order, plus bias and rounding.
+static void launch_sum(hipStream_t s, LinearArgs c, const float *part, uint32_t parts) {
+  c.groups = parts;
+  const dim3 grid((c.m * c.n + 255u) / 256u);
+  if (parts <= 8u)
+    k_linear_sum<8><<<grid, 256, 0, s>>>(c, part);
+  else if (parts <= 16u)
+    k_linear_sum<16><<<grid, 256, 0, s>>>(c, part);
+  else if (parts <= 32u)
+    k_linear_sum<32><<<grid, 256, 0, s>>>(c, part);
+  else
+    k_linear_sum<64><<<grid, 256, 0, s>>>(c, part);
+}
+
 // The tiled EXACT path, in token chunks whose group partials fit the
 // workspace (kLinPartBytes): tile kernel, then the ordered group sum.
 static hipError_t launch_exact_tiled(hipStream_t s, const LinearArgs &a, const LinearWorkspace &ws) {
@@ -1174,15 +1351,7 @@ static hipError_t launch_exact_tiled(hipStream_t s, const LinearArgs &a, const L
       launch_tile_mt<4>(s, c, ws.part);
     else
       launch_tile_mt<8>(s, c, ws.part);
-    const dim3 sum_grid((c.m * c.n + 255u) / 256u);
-    if (c.groups <= 8u)
-      k_linear_sum<8><<<sum_grid, 256, 0, s>>>(c, ws.part);
-    else if (c.groups <= 16u)
-      k_linear_sum<16><<<sum_grid, 256, 0, s>>>(c, ws.part);
-    else if (c.groups <= 32u)
-      k_linear_sum<32><<<sum_grid, 256, 0, s>>>(c, ws.part);
-    else
-      k_linear_sum<64><<<sum_grid, 256, 0, s>>>(c, ws.part);
+    launch_sum(s, c, ws.part, c.groups);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -1236,6 +1405,21 @@ static hipError_t launch_exact_mfma(hipStream_t s, const LinearArgs &a) {
   return hipGetLastError();
 }
 
+template <int TT>
+static void launch_gemm_tt(hipStream_t s, const LinearArgs &a, float *part, uint32_t splits) {
+  const uint32_t tok_blocks = (a.m + 16u * TT - 1u) / (16u * TT);
+  const uint32_t total = (a.n + kLgRows - 1u) / kLgRows * tok_blocks * splits;
+  const uint32_t grid = (total + 7u) / 8u * 8u, per = (a.groups + splits - 1u) / splits;
+  if (a.x_scale_f32 && a.w_scale_f32)
+    k_linear_gemm<TT, true, true><<<grid, 64 * kLgWaves, 0, s>>>(a, part, tok_blocks, total, per);
+  else if (a.x_scale_f32)
+    k_linear_gemm<TT, true, false><<<grid, 64 * kLgWaves, 0, s>>>(a, part, tok_blocks, total, per);
+  else if (a.w_scale_f32)
+    k_linear_gemm<TT, false, true><<<grid, 64 * kLgWaves, 0, s>>>(a, part, tok_blocks, total, per);
+  else
+    k_linear_gemm<TT, false, false><<<grid, 64 * kLgWaves, 0, s>>>(a, part, tok_blocks, total, per);
+}
+
 static hipError_t launch_exact_plan(hipStream_t s, const LinearArgs &a, const LinExactPlan &p) {
   switch (p.tokens * 100u + p.waves) {
     case 404u: return launch_exact_mfma<4, 1, 4>(s, a);
@@ -1264,6 +1448,20 @@ hipError_t launch_fp8_linear(hipStream_t s, const LinearArgs &a, int mode, const
     return hipGetLastError();
   }
   const bool fast = mode == S14_MODE_FAST && a.k % (4u * kLinGroup) == 0u;
+  // the prompt tiles from where they measured faster than k_linear_fast
+  // (us: wq_b m = 8 11.7 against 12.0, m = 12 17.9 against 11.9; wo_b m = 12 24.3
+  // against 13.8; wkv m = 64 14.6 against 17.8, m = 333 27.6 against 17.9)
+  if (fast && a.m > 8u && uint64_t(a.m) * a.n * a.k >= 300000000ull && uint64_t(a.n + kLgRows - 1) * a.k <= 0xFFFFFFFFull) {
+    const LinGemmPlan p = lin_gemm_plan(a.m, a.n, a.groups);
+    float *part = p.splits > 1u ? ws.part : nullptr;
+    if (p.tokens == 32u)
+      launch_gemm_tt<2>(s, a, part, p.splits);
+    else
+      launch_gemm_tt<4>(s, a, part, p.splits);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    if (part) launch_sum(s, a, part, p.splits);
+    return hipGetLastError();
+  }
   const LinFastPlan plan = fast ? lin_fast_plan(a.m, a.n, a.groups) : LinFastPlan{0, 0};
   if (plan.cw) {
     // one launch per plan.blocks token blocks, each within the workspace's

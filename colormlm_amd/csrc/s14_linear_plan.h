@@ -7,6 +7,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <initializer_list>
 
 namespace s14 {
 
@@ -68,6 +69,37 @@ inline LinFastPlan lin_fast_plan(uint32_t m, uint32_t n, uint32_t G) {
     if (blocks == 1) return {0, 0};
     blocks = (blocks + 1) / 2;
   }
+}
+
+// FAST for prompts (k_linear_gemm): 128 rows x `tokens` per workgroup, K in
+// `splits` ranges whose sums go through the workspace.  The split with the
+// least estimated time, in ns: a group of one workgroup takes 1,070 alone on
+// its CU and 1,600 when two share it (wo_a, wo_b at 512 tokens, 64 a
+// workgroup; the 32-token form a little over half); splits write and read
+// their sums at about 4 TB/s and take a second launch.
+struct LinGemmPlan {
+  uint32_t tokens, splits;
+};
+inline LinGemmPlan lin_gemm_plan(uint32_t m, uint32_t n, uint32_t G) {
+  const uint32_t tokens = m <= 32u ? 32u : 64u;
+  const uint64_t tiles = (uint64_t(n) + 127u) / 128u * ((uint64_t(m) + tokens - 1u) / tokens);
+  const uint64_t alone = tokens == 32u ? 650u : 1070u, shared = tokens == 32u ? 900u : 1600u;
+  LinGemmPlan best{tokens, 1};
+  uint64_t least = ~uint64_t(0);
+  for (uint32_t s : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u, 24u, 32u}) {
+    const uint64_t part = uint64_t(m) * n * s * sizeof(float), per = (G + s - 1u) / s;
+    // at least four groups a split (as k_linear_fast has: more partial sums
+    // round more often), and none without any
+    if (s > 1u && (part > kLinPartBytes || per < 4u || uint64_t(s - 1u) * per >= G)) continue;
+    const uint64_t wgs = tiles * s;
+    const uint64_t t = (wgs <= 256u ? alone : (wgs + 511u) / 512u * shared) * per +
+                       (s > 1u ? 3000u + 2u * part / 4000u : 0u);
+    if (t < least) {
+      least = t;
+      best.splits = s;
+    }
+  }
+  return best;
 }
 
 // EXACT on the f32 MFMA (k_linear_exact_mfma): tokens per workgroup and

@@ -283,6 +283,33 @@ def test_fp8_linear_exact_token_chunks(ctx, oracle):
     assert np.array_equal(host(y).view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("m,n,k,f32", [(9, 33000, 1024, False), (31, 8192, 1536, True), (33, 4099, 4096, False),
+                                       (64, 1030, 8192, True), (65, 8200, 1024, False), (200, 512, 4096, False),
+                                       (333, 700, 2560, True)])
+def test_fp8_linear_fast_prompt_tiles(ctx, oracle, m, n, k, f32):
+    """The prompt-tile FAST kernel: 32- and 64-token workgroups, rows cut by n
+    inside a wavefront's and a workgroup's rows (and n not a multiple of 4:
+    the scalar stores), tokens cut inside a block, K in one range and in
+    several (ragged ones too); f32 scales with a bias, and bf16 outputs."""
+    say(f"fp8_linear fast prompt tiles m={m} n={n} k={k} f32={f32}")
+    rng = np.random.default_rng(m + n)
+    w, x = codes(rng, (n, k)), codes(rng, (m, k))
+    if f32:
+        ws = rng.uniform(1e-3, 4e-3, (-(-n // 128), k // 128)).astype(np.float32)
+        xs = rng.uniform(1e-2, 3e-2, (m, k // 128)).astype(np.float32)
+    else:
+        ws = rng.integers(114, 122, (-(-n // 128), k // 128), dtype=np.uint8)
+        xs = rng.integers(120, 128, (m, k // 128), dtype=np.uint8)
+    b = rng.standard_normal(n).astype(np.float32) if f32 else np.zeros(n, np.float32)
+    want = oracle.fp8_linear(x, xs, w, ws, bias=b)
+    y = torch.full((m, n), np.nan, dtype=torch.float32, device="cuda")
+    s14.fp8_linear(ctx, dev(x), dev(xs), dev(w), dev(ws), y, bias=dev(b), mode=s14.FAST)
+    got = host(y)
+    check_fast(oracle, got - b, (want - b).astype(np.float64), x, xs, w, ws, f"m={m} n={n} k={k}")
+    s14.fp8_linear(ctx, dev(x), dev(xs), dev(w), dev(ws), y, bias=dev(b), round_bf16=True, mode=s14.FAST)
+    assert np.array_equal(host(y), torch.from_numpy(got).bfloat16().float().numpy())
+
+
 @pytest.mark.parametrize("m", [129, 512])
 def test_fp8_linear_fast_token_blocks_in_several_launches(ctx, oracle, m):
     """wq_b's FAST split-K partials take 8 MiB per 32-token block, so the
