@@ -96,16 +96,48 @@ __device__ __forceinline__ float chain_literal(float acc, const v2f (&q)[16], fl
   return acc;
 }
 using K32 = std::make_integer_sequence<int, 32>;
+// Official: x is an act_quant value (an e4m3 value times a power of two) and
+// the weight e2m1 or e4m3 times one, so the product has at most eight
+// significant bits: exact, and one fused multiply-add rounds like the
+// oracle's multiply and add.  32 instructions a group instead of 64.
+// x_k is the fused instruction's own DPP operand, written as asm: the
+// compiler keeps the broadcast as a move (and two wait states) per product.
+// The wait states ahead of each half cover a copy of x the compiler may
+// place there (a DPP read of a register a VALU instruction just wrote).
+__device__ __forceinline__ float chain_fma16(float acc, const v2f *q, float x) {
+#define S14_F(i) \
+  "v_fmac_f32_dpp %[acc], %[x], %[q" #i "] row_newbcast:" #i " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+  asm volatile("s_nop 1\n\t" S14_F(0) S14_F(1) S14_F(2) S14_F(3) S14_F(4) S14_F(5) S14_F(6) S14_F(7) S14_F(8) S14_F(9)
+                   S14_F(10) S14_F(11) S14_F(12) S14_F(13) S14_F(14) S14_F(15)
+               : [acc] "+v"(acc)
+               : [x] "v"(x), [q0] "v"(q[0].x), [q1] "v"(q[0].y), [q2] "v"(q[1].x), [q3] "v"(q[1].y),
+                 [q4] "v"(q[2].x), [q5] "v"(q[2].y), [q6] "v"(q[3].x), [q7] "v"(q[3].y), [q8] "v"(q[4].x),
+                 [q9] "v"(q[4].y), [q10] "v"(q[5].x), [q11] "v"(q[5].y), [q12] "v"(q[6].x), [q13] "v"(q[6].y),
+                 [q14] "v"(q[7].x), [q15] "v"(q[7].y));
+#undef S14_F
+  return acc;
+}
+__device__ __forceinline__ float chain_fma(float acc, const v2f (&q)[16], float xa, float xb) {
+  return chain_fma16(chain_fma16(acc, q, xa), q + 8, xb);
+}
+// The fused form also needs every product finite (the separate multiply
+// would round an overflow to infinity before the add): |x| < 2^(emax-126)
+// and |weight| <= 6 * 2^(c-127), or 448 * 2^(c-127) in FP8 rows.
+__device__ __forceinline__ CodeWindow fma_window(CodeWindow w) {
+  w.cmax = min(w.cmax, 376 - w.emax);
+  return w;
+}
 
 // FP8 rows (the reference's FP8 shared page): 32 code bytes per group, one
 // UE8M0 scale per 128 x 128 tile; p = (x * e4m3) * s
-// (s14_vulkan_numeric.rs:1698-1714), literal always.
-__device__ __forceinline__ void decode32_fp8(v2f (&q)[16], uint4 a, uint4 b) {
+// (s14_vulkan_numeric.rs:1698-1714): the scaled decode where the scale is in
+// fp8_code_in's window, else scale 1 and the literal two multiplies.
+__device__ __forceinline__ void decode32_fp8(v2f (&q)[16], uint4 a, uint4 b, float scale) {
   const uint32_t words[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
   for (int d = 0; d < 8; ++d) {
-    q[2 * d + 0] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(words[d], 1.0f, false);
-    q[2 * d + 1] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(words[d], 1.0f, true);
+    q[2 * d + 0] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(words[d], scale, false);
+    q[2 * d + 1] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(words[d], scale, true);
   }
 }
 
@@ -180,7 +212,7 @@ __device__ __forceinline__ uint32_t chunk_code(const ChunkRegs &cr, int i) {
 }
 
 // Consume chunk c from slot S: 8 groups of the lane's row, k ascending.
-template <int S>
+template <int S, bool kFma>
 __device__ __forceinline__ float chunk_consume(float acc, const ChunkRegs &cr, uint32_t wave, CodeWindow win,
                                                const RowStream &st, int c) {
   const uint32_t lane = threadIdx.x & 63;
@@ -197,7 +229,10 @@ __device__ __forceinline__ float chunk_consume(float acc, const ChunkRegs &cr, u
       const uint4 w = *reinterpret_cast<const uint4 *>(row + 16u * (uint32_t(i) ^ (lane & 7u)));
       v2f q[16];
       decode32(q, w, __uint_as_float(chunk_code(cr, i) << 23));
-      acc = chain_scaled(acc, q, cr.a[i], cr.b[i], K32{});
+      if constexpr (kFma)
+        acc = chain_fma(acc, q, cr.a[i], cr.b[i]);
+      else
+        acc = chain_scaled(acc, q, cr.a[i], cr.b[i], K32{});
     }
   } else {
     // literal decode (a code outside the window): group by group, codes from
@@ -219,7 +254,7 @@ __device__ __forceinline__ float chunk_consume(float acc, const ChunkRegs &cr, u
 }
 
 // Dot of the lane's MXFP4 row (NC chunks) with st.x, k ascending.
-template <int NC>
+template <int NC, bool kFma>
 __device__ __forceinline__ float row_dot_stream(const RowStream &st, uint32_t wave, CodeWindow win) {
   static_assert(NC % 2 == 0, "chunk pairs");
   ChunkRegs c0, c1;
@@ -230,22 +265,23 @@ __device__ __forceinline__ float row_dot_stream(const RowStream &st, uint32_t wa
   for (int c = 0; c < NC; c += 2) {
     stream_issue<1>(st, wave, c + 1);
     chunk_regs(c1, st, c + 1);
-    acc = chunk_consume<0>(acc, c0, wave, win, st, c);
+    acc = chunk_consume<0, kFma>(acc, c0, wave, win, st, c);
     if (c + 2 < NC) {
       stream_issue<0>(st, wave, c + 2);
       chunk_regs(c0, st, c + 2);
     }
-    acc = chunk_consume<1>(acc, c1, wave, win, st, c + 1);
+    acc = chunk_consume<1, kFma>(acc, c1, wave, win, st, c + 1);
   }
-  return acc;
+  return kFma ? asm_chain_end(acc) : acc;
 }
 
 // FP8 rows (the reference's FP8 shared page): 32 code bytes per group, one
 // UE8M0 scale per 128 x 128 tile; p = (x * e4m3) * s
-// (s14_vulkan_numeric.rs:1698-1714), literal always; rare (that variant's
-// shared page only), read straight from memory.
-template <int G>
-__device__ __forceinline__ float row_dot_fp8(Rsrc r, uint32_t woff, uint32_t soff_tiles, const float *x) {
+// (s14_vulkan_numeric.rs:1698-1714); rare (that variant's shared page
+// only), read straight from memory.
+template <int G, bool kFma>
+__device__ __forceinline__ float row_dot_fp8(Rsrc r, uint32_t woff, uint32_t soff_tiles, const float *x,
+                                             CodeWindow win) {
   float acc = 0.0f;
   const uint32_t j = threadIdx.x & 15u;
 #pragma unroll 1
@@ -259,15 +295,29 @@ __device__ __forceinline__ float row_dot_fp8(Rsrc r, uint32_t woff, uint32_t sof
       xa[i] = x[32 * (g0 + i) + j];
       xb[i] = x[32 * (g0 + i) + 16 + j];
     }
-    const float s = ue8m0_f32(ld1(r, soff_tiles + uint32_t(g0 / 4)));
+    const uint32_t code = ld1(r, soff_tiles + uint32_t(g0 / 4));
+    const bool ok = fp8_code_in(code, win) && (!kFma || int(code) <= 370 - win.emax);
+    if (__builtin_amdgcn_ballot_w64(!ok) == 0ull) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v2f q[16];
-      decode32_fp8(q, wa[i], wb[i]);
-      acc = chain_literal(acc, q, s, xa[i], xb[i], K32{});
+      for (int i = 0; i < 4; ++i) {
+        v2f q[16];
+        decode32_fp8(q, wa[i], wb[i], __uint_as_float(code << 23));
+        if constexpr (kFma)
+          acc = chain_fma(acc, q, xa[i], xb[i]);
+        else
+          acc = chain_scaled(acc, q, xa[i], xb[i], K32{});
+      }
+    } else {
+      const float s = ue8m0_f32(code);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v2f q[16];
+        decode32_fp8(q, wa[i], wb[i], 1.0f);
+        acc = chain_literal(acc, q, s, xa[i], xb[i], K32{});
+      }
     }
   }
-  return acc;
+  return kFma ? asm_chain_end(acc) : acc;
 }
 
 __device__ __forceinline__ uint32_t b_page_bytes(uint32_t fmt) {
@@ -310,6 +360,10 @@ __global__ __launch_bounds__(64 * kBWaves) void k_block_phase1(const PairTable *
   const bool upper = lane >= 32;
   const uint32_t row = row0 + (lane & 31u);
   const Rsrc r = make_rsrc(page, b_page_bytes(fmt));
+  // x's decode window: the exponent range the route kernel recorded
+  const uint32_t xw = uint32_t(__builtin_amdgcn_readlane(int(xw_all), int(t)));
+  CodeWindow win = mx_window(int(xw & 0xffffu), int(xw >> 16));
+  if constexpr (kOfficial) win = fma_window(win);
   float acc;
   if (fmt == S14_PAGE_MXFP4) {
     RowStream st;
@@ -322,13 +376,10 @@ __global__ __launch_bounds__(64 * kBWaves) void k_block_phase1(const PairTable *
       const uint32_t base = uint32_t(dr < 32 ? mx.w1 : mx.w3) + (row0 + (dr & 31u)) * (kHidden / 2);
       st.dma[j] = base + 16u * ((lane & 7u) ^ (dr & 7u));
     }
-    // x's decode window: the exponent range the route kernel recorded
-    const uint32_t xw = uint32_t(__builtin_amdgcn_readlane(int(xw_all), int(t)));
-    const CodeWindow win = mx_window(int(xw & 0xffffu), int(xw >> 16));
-    acc = row_dot_stream<kHidden / 32 / kBChunk>(st, wave, win);
+    acc = row_dot_stream<kHidden / 32 / kBChunk, kOfficial>(st, wave, win);
   } else {
-    acc = row_dot_fp8<kHidden / 32>(r, uint32_t(upper ? f8.w3 : f8.w1) + row * kHidden,
-                                    uint32_t(upper ? f8.s3 : f8.s1) + (row / 128) * (kHidden / 128), x);
+    acc = row_dot_fp8<kHidden / 32, kOfficial>(r, uint32_t(upper ? f8.w3 : f8.w1) + row * kHidden,
+                                               uint32_t(upper ? f8.s3 : f8.s1) + (row / 128) * (kHidden / 128), x, win);
   }
   const float u = lane_xor32(acc);
   int lo = 255, hi = 0;
@@ -381,6 +432,8 @@ __global__ __launch_bounds__(64 * kBWaves) void k_block_phase2(const PairTable *
   const uint32_t row0 = (q * kBWaves + wave) * kBRowsW;
   const uint32_t row = row0 + lane;
   const Rsrc r = make_rsrc(page, b_page_bytes(fmt));
+  CodeWindow win = mx_window(wave_min_i(int(wrec & 0xffffu)), wave_max_i(int(wrec >> 16)));
+  if constexpr (kOfficial) win = fma_window(win);
   float acc;
   if (fmt == S14_PAGE_MXFP4) {
     RowStream st;
@@ -392,11 +445,10 @@ __global__ __launch_bounds__(64 * kBWaves) void k_block_phase2(const PairTable *
       const uint32_t dr = 8u * j + (lane >> 3);
       st.dma[j] = uint32_t(mx.w2) + (row0 + dr) * (kInter / 2) + 16u * ((lane & 7u) ^ (dr & 7u));
     }
-    const CodeWindow win = mx_window(wave_min_i(int(wrec & 0xffffu)), wave_max_i(int(wrec >> 16)));
-    acc = row_dot_stream<kInter / 32 / kBChunk>(st, wave, win);
+    acc = row_dot_stream<kInter / 32 / kBChunk, kOfficial>(st, wave, win);
   } else {
-    acc = row_dot_fp8<kInter / 32>(r, uint32_t(f8.w2) + row * kInter, uint32_t(f8.s2) + (row / 128) * (kInter / 128),
-                                   h);
+    acc = row_dot_fp8<kInter / 32, kOfficial>(r, uint32_t(f8.w2) + row * kInter,
+                                              uint32_t(f8.s2) + (row / 128) * (kInter / 128), h, win);
   }
   if constexpr (kOfficial) acc = bf16_round(acc);
   ws.down[size_t(p) * kHidden + row] = acc;

@@ -975,9 +975,12 @@ __global__ __launch_bounds__(64 * kP1ExactWaves) void k_phase1_exact(PairTable p
   } else {
     const uint32_t woff = uint32_t(upper ? f8.w3 : f8.w1) + row * kHidden + 16u * h;
     const uint32_t soff = uint32_t(upper ? f8.s3 : f8.s1) + (row / 128) * (kHidden / 128);
-    stage_x_block<kHidden, 64 * kP1ExactWaves>(xs, srcx, red);
-    if constexpr (kOfficial && !kXq) requant128_block<64 * kP1ExactWaves>(xs, kHidden, red);
-    acc = fp8_row_pair(0.0f, src, woff, soff, 0, kHidden / 32, xs + 16 * h);
+    Fp8Batch8 ba;
+    fp8_load8(ba, src, woff, soff, 0);  // as above: first weights and the row's codes ahead of the x copy
+    const uint32_t code = fp8_row_code<kHidden / 32>(src, soff);
+    CodeWindow win = stage_x_block<kHidden, 64 * kP1ExactWaves>(xs, srcx, red);
+    if constexpr (kOfficial && !kXq) win = requant128_block<64 * kP1ExactWaves>(xs, kHidden, red);
+    acc = fp8_row_pair_fixed<kHidden / 32>(ba, src, woff, soff, xs + 16 * h, win, code);
   }
   const float other = lane_xor32(acc);
   const bool writer = !upper && h == 0;
@@ -1219,6 +1222,19 @@ __global__ __launch_bounds__(64 * kP2ExactWaves) void k_phase2_exact(const PairT
     mx_load<kPF>(ba, srcp, mx_woff, mx_soff, 0);  // first weights and the row's codes in flight during the h copy
     load_row_codes<kInter / 32>(rc, srcp, mx_soff);
   }
+  // an FP8 page alone in its wavefront (the shared page is a token's last
+  // slot, so it is unless the token has an odd number of routed pairs): one
+  // page for all lanes, the same prefetch
+  const bool f8_alone = has_a && !has_b && fa == S14_PAGE_FP8;
+  const uint32_t f8_woff = uint32_t(f8.w2) + row * kInter + 16u * h;
+  const uint32_t f8_soff = uint32_t(f8.s2) + (row / 128) * (kInter / 128);
+  const Src1 src8{src.a, src.a};
+  Fp8Batch8 b8;
+  uint32_t code8 = 0;
+  if (f8_alone) {
+    fp8_load8(b8, src8, f8_woff, f8_soff, 0);
+    code8 = fp8_row_code<kInter / 32>(src8, f8_soff);
+  }
   // h loads first, then the window words (whose reduction waits for them)
   CodeWindow win[2] = {{256, 0}, {256, 0}};
   if (has_b) {
@@ -1243,13 +1259,14 @@ __global__ __launch_bounds__(64 * kP2ExactWaves) void k_phase2_exact(const PairT
     float acc;
     if (fa == S14_PAGE_MXFP4 && fb == S14_PAGE_MXFP4) {
       acc = mx_row_pair_fixed<kPF, kInter / 32>(0.0f, ba, srcp, mx_woff, mx_soff, xh, (hi ? win[1] : win[0]), rc);
+    } else if (f8_alone) {
+      acc = fp8_row_pair_fixed<kInter / 32>(b8, src8, f8_woff, f8_soff, xh, win[0], code8);
     } else if (mine_mx) {  // formats differ between the halves
       MxBatch<kPF> bm;
       mx_load<kPF>(bm, src, mx_woff, mx_soff, 0);
       acc = mx_row_pair<kPF>(0.0f, bm, src, mx_woff, mx_soff, kInter / 32, xh, (hi ? win[1] : win[0]));
     } else {
-      acc = fp8_row_pair(0.0f, src, uint32_t(f8.w2) + row * kInter + 16u * h,
-                         uint32_t(f8.s2) + (row / 128) * (kInter / 128), 0, kInter / 32, xh);
+      acc = fp8_row_pair(0.0f, src, f8_woff, f8_soff, 0, kInter / 32, xh);
     }
     if constexpr (kOfficial) acc = bf16_round(acc);  // w2's output rounded to bf16
     if (h == 0 && (!hi || has_b)) part[slot][r] = acc;
