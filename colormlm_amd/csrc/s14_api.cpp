@@ -505,11 +505,15 @@ int block_route_launch(hipStream_t st, const Workspace &ws, uint32_t tokens, con
   if (e != hipSuccess) return hip_fail(e, "router launch");
   if (tokens > 1 && (mode == S14_MODE_EXACT || official)) {
     // blocks: one row per lane (enough (token, expert) chains to fill the
-    // GPU).  With a side stream the pairs run as two halves, one per stream,
-    // so that the SIMDs one half's phase-1 tail leaves idle (3.5 equal
+    // GPU).  With a side stream the pairs can run as two halves, one per
+    // stream, so that the SIMDs one half's phase-1 tail leaves idle (3.5 equal
     // wavefronts per SIMD, two resident at a time) take the other half's
-    // work: K=8 182.9 -> 170.7 us per block (an even split measured best; three
-    // or four streams were slower).  Stage events time the first half.
+    // work.  The fork and the join cost about 18 us of event latency, so it
+    // pays only for the longest blocks (us, one stream against two: EXACT
+    // T = 2 61.5 / 95.8, 4 98.0 / 108.4, 6 135.2 / 143.3, 7 163.3 / 160.3, 8 170.9 /
+    // 168.1; official T = 8 158.5 / 161.9).  An even split measured best; three
+    // or four streams were slower.  Stage events time the first half.
+    if (official || tokens < 7) fork = nullptr;
     const uint32_t na = fork ? n_pairs / 2 : n_pairs, nb = n_pairs - na;
     if (fork) {
       if ((e = hipEventRecord(fork->fork, st)) != hipSuccess) return hip_fail(e, "hipEventRecord(fork)");

@@ -102,23 +102,77 @@ using K32 = std::make_integer_sequence<int, 32>;
 // oracle's multiply and add.  32 instructions a group instead of 64.
 // x_k is the fused instruction's own DPP operand, written as asm: the
 // compiler keeps the broadcast as a move (and two wait states) per product.
-// The wait states ahead of each half cover a copy of x the compiler may
-// place there (a DPP read of a register a VALU instruction just wrote).
-__device__ __forceinline__ float chain_fma16(float acc, const v2f *q, float x) {
+// A chain's fused adds wait about nine cycles for one another, so each half
+// group's 16 carry the next half's eight conversions in their gaps (the
+// compiler puts the conversions, and the LDS read before them, in a run of
+// their own ahead of each group).  Two instructions stand ahead of the first
+// DPP read: the wait states a copy of x placed there by the compiler needs.
 #define S14_F(i) \
-  "v_fmac_f32_dpp %[acc], %[x], %[q" #i "] row_newbcast:" #i " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+  "v_fmac_f32_dpp %[acc], %[x], %[p" #i "] row_newbcast:" #i " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+#define S14_FMA_IN                                                                                                  \
+  [x] "v"(x), [p0] "v"(p[0].x), [p1] "v"(p[0].y), [p2] "v"(p[1].x), [p3] "v"(p[1].y), [p4] "v"(p[2].x),             \
+      [p5] "v"(p[2].y), [p6] "v"(p[3].x), [p7] "v"(p[3].y), [p8] "v"(p[4].x), [p9] "v"(p[4].y), [p10] "v"(p[5].x), \
+      [p11] "v"(p[5].y), [p12] "v"(p[6].x), [p13] "v"(p[6].y), [p14] "v"(p[7].x), [p15] "v"(p[7].y)
+#define S14_CVT_OUT                                                                                             \
+  [q0] "=&v"(q[0]), [q1] "=&v"(q[1]), [q2] "=&v"(q[2]), [q3] "=&v"(q[3]), [q4] "=&v"(q[4]), [q5] "=&v"(q[5]), \
+      [q6] "=&v"(q[6]), [q7] "=&v"(q[7])
+#define S14_FMA_CVT(C0, C1, C2, C3, C4, C5, C6, C7)                                                            \
+  C0 C1 S14_F(0) S14_F(1) C2 S14_F(2) S14_F(3) C3 S14_F(4) S14_F(5) C4 S14_F(6) S14_F(7) C5 S14_F(8) S14_F(9) \
+      C6 S14_F(10) S14_F(11) C7 S14_F(12) S14_F(13) S14_F(14) S14_F(15)
+// acc + the half's 16 products x_k * p_k in order; q: the 16 values of the
+// MXFP4 codes w (two words) times sc.
+__device__ __forceinline__ float chain_fma16_mx(float acc, float x, const v2f *p, v2f *q, uint32_t w0, uint32_t w1,
+                                                float sc) {
+#define S14_C(d, w, sel) "v_cvt_scalef32_pk_f32_fp4 %[q" #d "], %[" #w "], %[sc]" sel "\n\t"
+  asm volatile(S14_FMA_CVT(S14_C(0, w0, ""), S14_C(1, w0, " op_sel:[1,0,0]"), S14_C(2, w0, " op_sel:[0,1,0]"),
+                           S14_C(3, w0, " op_sel:[1,1,0]"), S14_C(4, w1, ""), S14_C(5, w1, " op_sel:[1,0,0]"),
+                           S14_C(6, w1, " op_sel:[0,1,0]"), S14_C(7, w1, " op_sel:[1,1,0]"))
+               : [acc] "+v"(acc), S14_CVT_OUT
+               : S14_FMA_IN, [w0] "v"(w0), [w1] "v"(w1), [sc] "v"(sc));
+#undef S14_C
+  return acc;
+}
+// The same with e4m3 codes (four words).
+__device__ __forceinline__ float chain_fma16_fp8(float acc, float x, const v2f *p, v2f *q, uint4 w, float sc) {
+#define S14_C(d, w, sel) "v_cvt_scalef32_pk_f32_fp8 %[q" #d "], %[" #w "], %[sc]" sel "\n\t"
+  asm volatile(S14_FMA_CVT(S14_C(0, w0, ""), S14_C(1, w0, " op_sel:[1,0,0]"), S14_C(2, w1, ""),
+                           S14_C(3, w1, " op_sel:[1,0,0]"), S14_C(4, w2, ""), S14_C(5, w2, " op_sel:[1,0,0]"),
+                           S14_C(6, w3, ""), S14_C(7, w3, " op_sel:[1,0,0]"))
+               : [acc] "+v"(acc), S14_CVT_OUT
+               : S14_FMA_IN, [w0] "v"(w.x), [w1] "v"(w.y), [w2] "v"(w.z), [w3] "v"(w.w), [sc] "v"(sc));
+#undef S14_C
+  return acc;
+}
+// A last half, with nothing to convert.
+__device__ __forceinline__ float chain_fma16(float acc, float x, const v2f *p) {
   asm volatile("s_nop 1\n\t" S14_F(0) S14_F(1) S14_F(2) S14_F(3) S14_F(4) S14_F(5) S14_F(6) S14_F(7) S14_F(8) S14_F(9)
                    S14_F(10) S14_F(11) S14_F(12) S14_F(13) S14_F(14) S14_F(15)
                : [acc] "+v"(acc)
-               : [x] "v"(x), [q0] "v"(q[0].x), [q1] "v"(q[0].y), [q2] "v"(q[1].x), [q3] "v"(q[1].y),
-                 [q4] "v"(q[2].x), [q5] "v"(q[2].y), [q6] "v"(q[3].x), [q7] "v"(q[3].y), [q8] "v"(q[4].x),
-                 [q9] "v"(q[4].y), [q10] "v"(q[5].x), [q11] "v"(q[5].y), [q12] "v"(q[6].x), [q13] "v"(q[6].y),
-                 [q14] "v"(q[7].x), [q15] "v"(q[7].y));
-#undef S14_F
+               : S14_FMA_IN);
   return acc;
 }
-__device__ __forceinline__ float chain_fma(float acc, const v2f (&q)[16], float xa, float xb) {
-  return chain_fma16(chain_fma16(acc, q, xa), q + 8, xb);
+#undef S14_FMA_CVT
+#undef S14_CVT_OUT
+#undef S14_FMA_IN
+#undef S14_F
+// The first half of a group's values (k 0..15), ahead of a run of halves.
+__device__ __forceinline__ void decode16_mx(v2f *q, uint32_t w0, uint32_t w1, float sc) {
+  const uint32_t words[2] = {w0, w1};
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    q[4 * d + 0] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(words[d], sc, 0);
+    q[4 * d + 1] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(words[d], sc, 1);
+    q[4 * d + 2] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(words[d], sc, 2);
+    q[4 * d + 3] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(words[d], sc, 3);
+  }
+}
+__device__ __forceinline__ void decode16_fp8(v2f *q, uint4 w, float sc) {
+  const uint32_t words[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    q[2 * d + 0] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(words[d], sc, false);
+    q[2 * d + 1] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(words[d], sc, true);
+  }
 }
 // The fused form also needs every product finite (the separate multiply
 // would round an overflow to infinity before the add): |x| < 2^(emax-126)
@@ -224,15 +278,29 @@ __device__ __forceinline__ float chunk_consume(float acc, const ChunkRegs &cr, u
     ok = ok && code >= win.cmin && code <= win.cmax;
   }
   if (__builtin_amdgcn_ballot_w64(!ok) == 0ull) {
+    if constexpr (kFma) {
+      uint4 w = *reinterpret_cast<const uint4 *>(row + 16u * (lane & 7u));
+      v2f qa[8], qb[8];
+      decode16_mx(qa, w.x, w.y, __uint_as_float(chunk_code(cr, 0) << 23));
 #pragma unroll
-    for (int i = 0; i < kBChunk; ++i) {
-      const uint4 w = *reinterpret_cast<const uint4 *>(row + 16u * (uint32_t(i) ^ (lane & 7u)));
-      v2f q[16];
-      decode32(q, w, __uint_as_float(chunk_code(cr, i) << 23));
-      if constexpr (kFma)
-        acc = chain_fma(acc, q, cr.a[i], cr.b[i]);
-      else
+      for (int i = 0; i < kBChunk; ++i) {
+        const float sc = __uint_as_float(chunk_code(cr, i) << 23);
+        const uint4 cur = w;
+        if (i + 1 < kBChunk) w = *reinterpret_cast<const uint4 *>(row + 16u * (uint32_t(i + 1) ^ (lane & 7u)));
+        acc = chain_fma16_mx(acc, cr.a[i], qa, qb, cur.z, cur.w, sc);
+        if (i + 1 < kBChunk)
+          acc = chain_fma16_mx(acc, cr.b[i], qb, qa, w.x, w.y, __uint_as_float(chunk_code(cr, i + 1) << 23));
+        else
+          acc = chain_fma16(acc, cr.b[i], qb);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < kBChunk; ++i) {
+        const uint4 w = *reinterpret_cast<const uint4 *>(row + 16u * (uint32_t(i) ^ (lane & 7u)));
+        v2f q[16];
+        decode32(q, w, __uint_as_float(chunk_code(cr, i) << 23));
         acc = chain_scaled(acc, q, cr.a[i], cr.b[i], K32{});
+      }
     }
   } else {
     // literal decode (a code outside the window): group by group, codes from
@@ -261,17 +329,22 @@ __device__ __forceinline__ float row_dot_stream(const RowStream &st, uint32_t wa
   stream_issue<0>(st, wave, 0);
   chunk_regs(c0, st, 0);
   float acc = 0.0f;
+  // the last two chunks peeled: with a conditional refill the compiler has
+  // to assume that it was not issued, so its wait for a chunk's x and codes
+  // also waited for the refill's loads, a memory latency every second chunk
 #pragma unroll 1
-  for (int c = 0; c < NC; c += 2) {
+  for (int c = 0; c < NC - 2; c += 2) {
     stream_issue<1>(st, wave, c + 1);
     chunk_regs(c1, st, c + 1);
     acc = chunk_consume<0, kFma>(acc, c0, wave, win, st, c);
-    if (c + 2 < NC) {
-      stream_issue<0>(st, wave, c + 2);
-      chunk_regs(c0, st, c + 2);
-    }
+    stream_issue<0>(st, wave, c + 2);
+    chunk_regs(c0, st, c + 2);
     acc = chunk_consume<1, kFma>(acc, c1, wave, win, st, c + 1);
   }
+  stream_issue<1>(st, wave, NC - 1);
+  chunk_regs(c1, st, NC - 1);
+  acc = chunk_consume<0, kFma>(acc, c0, wave, win, st, NC - 2);
+  acc = chunk_consume<1, kFma>(acc, c1, wave, win, st, NC - 1);
   return kFma ? asm_chain_end(acc) : acc;
 }
 
@@ -298,14 +371,22 @@ __device__ __forceinline__ float row_dot_fp8(Rsrc r, uint32_t woff, uint32_t sof
     const uint32_t code = ld1(r, soff_tiles + uint32_t(g0 / 4));
     const bool ok = fp8_code_in(code, win) && (!kFma || int(code) <= 370 - win.emax);
     if (__builtin_amdgcn_ballot_w64(!ok) == 0ull) {
+      const float sc = __uint_as_float(code << 23);
+      if constexpr (kFma) {
+        v2f qa[8], qb[8];
+        decode16_fp8(qa, wa[0], sc);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v2f q[16];
-        decode32_fp8(q, wa[i], wb[i], __uint_as_float(code << 23));
-        if constexpr (kFma)
-          acc = chain_fma(acc, q, xa[i], xb[i]);
-        else
+        for (int i = 0; i < 4; ++i) {
+          acc = chain_fma16_fp8(acc, xa[i], qa, qb, wb[i], sc);
+          acc = i < 3 ? chain_fma16_fp8(acc, xb[i], qb, qa, wa[i + 1 < 4 ? i + 1 : i], sc) : chain_fma16(acc, xb[i], qb);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          v2f q[16];
+          decode32_fp8(q, wa[i], wb[i], sc);
           acc = chain_scaled(acc, q, xa[i], xb[i], K32{});
+        }
       }
     } else {
       const float s = ue8m0_f32(code);

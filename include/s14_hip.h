@@ -274,7 +274,7 @@ int s14_moe_layer_route(s14_ctx *ctx, void *stream, const s14_router *router,
  * layer, grouped expert-major so each distinct expert page is read once per
  * block.  ids_out [T, topk] u16 and weights_out [T, topk] f32 (device, may be
  * NULL); s14_last_block_distinct reports the distinct routed page count.
- * An EXACT block of T >= 2 runs half of its pairs on the context's own side
+ * An EXACT block of T >= 7 runs half of its pairs on the context's own side
  * stream, joined back into `stream` (event wait) before the output is
  * written: work queued on `stream` afterwards sees y complete, and a graph
  * capture of `stream` takes the side branch in. */

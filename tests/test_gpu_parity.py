@@ -1240,6 +1240,44 @@ def test_official_route_given_fp8_shared(ctx, oracle, bank):
     assert_bit_exact(host(y), want, "official fp8 shared")
 
 
+@pytest.mark.parametrize("mode", [s14.EXACT, s14.OFFICIAL])
+@pytest.mark.parametrize("topk", [6, 5])
+def test_fp8_shared_edge_scale_codes(ctx, oracle, bank, mode, topk):
+    """FP8 shared pages with tile scale codes outside the scaled decode's
+    window (0..9 in some tiles of w1, w3 and w2: the literal two multiplies)
+    beside ordinary ones, the shared slot alone in its phase-2 wavefront
+    (topk 6) and beside a routed one (topk 5); a layer with the route given
+    whose x also holds tiny and zero values, and a block of 3."""
+    say(f"FP8 shared page with edge tile scales, mode={mode} topk={topk}")
+    o = synth.page_offsets("fp8")
+    sh = synth.gen_fp8_page(0, 0).copy()
+    sh[o["s1"] + 3 * 32 + 7], sh[o["s1"] + 5 * 32] = 0, 9
+    sh[o["s3"] + 9 * 32 + 31], sh[o["s3"] + 3 * 32 + 8] = 4, 1
+    sh[o["s2"] + 2 * 16 + 15], sh[o["s2"] + 30 * 16] = 0, 8
+    layer = oracle.moe_layer_official if mode == s14.OFFICIAL else oracle.moe_layer
+    ids = [126, 12, 205, 149, 227, 174][:topk]
+    w = np.array([0.3, 0.2, 0.15, 0.15, 0.1, 0.1], dtype=np.float32)[:topk]
+    y = torch.empty(HIDDEN, dtype=torch.float32, device="cuda")
+    for tiny in (False, True):
+        x = synth.token(seed=3)
+        if tiny:
+            x[5], x[300], x[4000] = np.float32(1e-39), np.float32(0.0), np.float32(-2e-37)
+        want = layer(x, [page_host(bank, e) for e in ids], w, sh, shared_fmt="fp8")
+        s14.moe_layer(ctx, [bank["pages"][e] for e in ids], w.tolist(), dev(sh), dev(x), y,
+                      shared_format=N.S14_PAGE_FP8, mode=mode)
+        assert_bit_exact(host(y), want, f"layer, tiny x {tiny}")
+    if topk == 6:
+        xs = synth.block_tokens(seed=15, tokens=3)
+        yb = torch.empty((3, HIDDEN), dtype=torch.float32, device="cuda")
+        s14.moe_block_route(ctx, 3, s14.Router(bank["wr_d"], bank["bias_d"]), bank["table"], dev(sh), dev(xs), yb,
+                            shared_format=N.S14_PAGE_FP8, mode=mode)
+        got = host(yb)
+        for t in range(3):
+            _, i_o, w_o = oracle.route(bank["wr"], bank["bias"], xs[t])
+            want = layer(xs[t], [page_host(bank, int(e)) for e in i_o], w_o, sh, shared_fmt="fp8")
+            assert_bit_exact(got[t], want, f"block token {t}")
+
+
 def test_official_chain_weight_before_w2(ctx, oracle, bank):
     """The expert chain in official mode: one routed expert, its weight on h
     before w2, no shared expert."""
