@@ -958,7 +958,8 @@ __global__ __launch_bounds__(64 * kGxWaves) void k_linear_gemv_exact(LinearArgs 
   const float sb = kWsF32 ? ldf(rsw, 4u * si) : ue8m0_f32(cw);
   // UE8M0 scales whose every a, b and a * b stays normal or zero (|dec| in
   // [2^-9, 448]): the converters' scale operand forms a and b exactly, the
-  // same values as the separate multiplies
+  // same values as the separate multiplies, and their product, of at most
+  // eight significant bits, is exact: one fused multiply-add per k
   const bool scaled = !kXsF32 && !kWsF32 && cx >= 10u && cx <= 246u && cw >= 10u && cw <= 246u &&
                       cx + cw >= 146u && cx + cw <= 364u;
   const uint8_t *wp = gx_w[wave] + r * K + kLinGroup * g;
@@ -991,7 +992,8 @@ __global__ __launch_bounds__(64 * kGxWaves) void k_linear_gemv_exact(LinearArgs 
           bv[0] = __fmul_rn(wl.x, sb), bv[1] = __fmul_rn(wl.y, sb), bv[2] = __fmul_rn(wh.x, sb), bv[3] = __fmul_rn(wh.y, sb);
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) partial = __fadd_rn(partial, __fmul_rn(av[e], bv[e]));  // k ascending
+        for (int e = 0; e < 4; ++e)  // k ascending
+          partial = kScaled ? fmaf(av[e], bv[e], partial) : __fadd_rn(partial, __fmul_rn(av[e], bv[e]));
       }
     }
   };
