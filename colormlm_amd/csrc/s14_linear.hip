@@ -1503,8 +1503,18 @@ hipError_t launch_fp8_linear(hipStream_t s, const LinearArgs &a, int mode, const
   // past 4,096 stay on the tiles below (wo_b m = 4: 21.5 us against 24.1:
   // 64-row workgroups leave most CUs idle there)
   if (vec && a.k % kLinGroup == 0u && !a.x_scale_f32 && !a.w_scale_f32 && (a.m > 4u || a.k <= 4096u) &&
-      uint64_t(a.n + kXmRows - 1) * a.k <= 0xFFFFFFFFull)
-    return launch_exact_plan(s, a, lin_exact_plan(a.m, a.n, a.groups));
+      uint64_t(a.n + kXmRows - 1) * a.k <= 0xFFFFFFFFull) {
+    const uint32_t first = lin_exact_first(a.m, a.n, a.groups);
+    LinearArgs c = a;
+    c.m = first;
+    const hipError_t e = launch_exact_plan(s, c, lin_exact_plan(c.m, c.n, c.groups));
+    if (e != hipSuccess || first == a.m) return e;
+    c.m = a.m - first;
+    c.x = a.x + size_t(first) * a.k;
+    c.x_scale = static_cast<const uint8_t *>(a.x_scale) + size_t(first) * a.groups;
+    c.y = a.y + size_t(first) * a.n;
+    return launch_exact_plan(s, c, lin_exact_plan(c.m, c.n, c.groups));
+  }
   // tiled: whole groups, one token's partials within the workspace, and the
   // last tile's row offsets within 32 bits (rows past n read zeros)
   if (vec && a.k % kLinGroup == 0u && size_t(a.groups) * a.n * sizeof(float) <= kLinPartBytes &&

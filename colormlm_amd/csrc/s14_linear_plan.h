@@ -111,6 +111,7 @@ inline LinGemmPlan lin_gemm_plan(uint32_t m, uint32_t n, uint32_t G) {
 // reads uncovered, many small ones convert the same weights more often.
 struct LinExactPlan {
   uint32_t tokens, waves;
+  uint64_t ns;  // estimated
 };
 inline LinExactPlan lin_exact_plan(uint32_t m, uint32_t n, uint32_t G) {
   struct Kind {
@@ -119,18 +120,33 @@ inline LinExactPlan lin_exact_plan(uint32_t m, uint32_t n, uint32_t G) {
   constexpr Kind kinds[] = {{4, 4, 1760, 1110},  {4, 16, 1220, 1420}, {8, 4, 3000, 1900},  {8, 8, 2400, 2500},
                             {16, 4, 3200, 2600}, {16, 8, 2650, 2850}, {32, 4, 5300, 4660}};
   const uint64_t tiles = (uint64_t(n) + 63u) / 64u;
-  LinExactPlan best{0, 0};
-  uint64_t least = ~uint64_t(0);
+  LinExactPlan best{0, 0, ~uint64_t(0)};
   for (const Kind &k : kinds) {
     const uint64_t wgs = tiles * ((uint64_t(m) + k.tokens - 1u) / k.tokens);
     const uint64_t t = (wgs + 255u) / 256u * ((G + k.waves - 1u) / k.waves) * (k.waves / 4u) *
                        (wgs <= 256u ? k.alone_ns : k.shared_ns);
-    if (t < least) {
-      least = t;
-      best = {k.tokens, k.waves};
-    }
+    if (t < best.ns) best = {k.tokens, k.waves, t};
   }
   return best;
+}
+// Tokens of a first launch when two launches (whole 32-token blocks, then
+// the rest) are estimated faster than one, else m: a last round of a few
+// workgroups costs as much as a full one (wo_a at 333 tokens: 11 blocks of 128
+// workgroups are 5.5 rounds, run as 6; 10 blocks and 13 tokens on their own
+// 214 us against 224).
+constexpr uint64_t kLinLaunchNs = 5000;
+inline uint32_t lin_exact_first(uint32_t m, uint32_t n, uint32_t G) {
+  uint64_t least = lin_exact_plan(m, n, G).ns;
+  uint32_t first = m;
+  for (uint32_t cut = m / 32u * 32u, i = 0; cut > 0u && i < 8u; cut -= 32u, ++i) {
+    if (cut == m) continue;
+    const uint64_t t = lin_exact_plan(cut, n, G).ns + lin_exact_plan(m - cut, n, G).ns + kLinLaunchNs;
+    if (t < least) {
+      least = t;
+      first = cut;
+    }
+  }
+  return first;
 }
 
 }  // namespace s14

@@ -241,10 +241,11 @@ def test_fp8_linear_exact_one_token_extreme_scales(ctx, oracle, k):
 @pytest.mark.parametrize("m,n,k", [(2, 300, 384), (3, 64, 128), (5, 4160, 1152), (7, 129, 4096), (13, 1000, 640),
                                    (17, 8192, 256), (31, 2000, 1536), (33, 16450, 512), (65, 700, 2176),
                                    (97, 8200, 384), (160, 12288, 256),
-                                   (52, 4160, 640), (132, 1000, 640), (12, 8192, 2048)])
+                                   (52, 4160, 640), (132, 1000, 640), (12, 8192, 2048),
+                                   (65, 8192, 2048)])
 def test_fp8_linear_exact_mfma_plans(ctx, oracle, m, n, k):
     """The f32-MFMA EXACT kernel with every plan (4, 8, 16 and 32 tokens per
-    workgroup; 4, 8 and 16 wavefronts): rows cut inside a 64-row tile,
+    workgroup; 4, 8 and 16 wavefronts; m = 65 in two launches): rows cut inside a 64-row tile,
     tokens cut inside a block, fewer groups than wavefronts and a ragged last
     round of groups; then UE8M0 codes that leave the MFMA's window (0..12, so
     that products fall to subnormals or zero), a bias and bf16 outputs; bit
