@@ -39,9 +39,7 @@ def _ptr(t) -> int:
 
 
 def _nbytes(t) -> int:
-    if hasattr(t, "untyped_storage"):
-        return int(t.numel() * t.element_size())
-    return int(t.nbytes)
+    return int(t.nbytes)  # elements times element size, for tensors and arrays alike
 
 
 def buffer(t, nbytes: Optional[int] = None) -> N.Buffer:
@@ -49,6 +47,17 @@ def buffer(t, nbytes: Optional[int] = None) -> N.Buffer:
     if t is None:
         return N.Buffer(None, 0)
     return N.Buffer(_ptr(t), _nbytes(t) if nbytes is None else nbytes)
+
+
+_SCALE_DTYPES = {}  # element type -> S14_SCALE_* (two tensor-to-text conversions a call otherwise)
+
+
+def _scale_dtype(t) -> int:
+    code = _SCALE_DTYPES.get(t.dtype)
+    if code is None:
+        code = N.S14_SCALE_F32 if str(t.dtype).endswith("float32") else N.S14_SCALE_UE8M0
+        _SCALE_DTYPES[t.dtype] = code
+    return code
 
 
 _TORCH_CUDA = []  # [torch] once torch with a visible GPU is found, [None] if not
@@ -64,11 +73,15 @@ def _stream(stream):
         try:
             import torch
 
+            if torch.cuda.is_available():
+                torch.cuda.init()  # before the raw stream is asked for below
             _TORCH_CUDA.append(torch if torch.cuda.is_available() else None)
         except Exception:  # pragma: no cover - torch is optional for the ABI
             _TORCH_CUDA.append(None)
     torch = _TORCH_CUDA[0]
-    return torch.cuda.current_stream().cuda_stream if torch is not None else None
+    if torch is None:
+        return None
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())  # current_stream().cuda_stream without the object
 
 
 class Context:
@@ -547,17 +560,14 @@ def fp8_linear(
     """fp8_linear (fp8.py:111-193): x e4m3 codes [m, k] (uint8), weight
     [n, k]; scales uint8 UE8M0 codes or float32, [m, ceil(k/128)] and
     [ceil(n/128), ceil(k/128)]; y float32 [m, n]."""
-    m, k = (1, x.shape[0]) if x.dim() == 1 else (x.shape[0], x.shape[-1])
+    shape = x.shape
+    m, k = (1, shape[0]) if len(shape) == 1 else (shape[0], shape[-1])
     n = weight.shape[0]
-
-    def sdt(t):
-        return N.S14_SCALE_F32 if str(t.dtype).endswith("float32") else N.S14_SCALE_UE8M0
-
     flags = N.S14_LINEAR_ROUND_BF16 if round_bf16 else 0
     check(
         lib().s14_fp8_linear(
-            ctx.handle, _stream(stream), m, n, k, buffer(x), buffer(x_scale), sdt(x_scale), buffer(weight),
-            buffer(weight_scale), sdt(weight_scale), buffer(bias), buffer(y), flags, mode
+            ctx.handle, _stream(stream), m, n, k, buffer(x), buffer(x_scale), _scale_dtype(x_scale), buffer(weight),
+            buffer(weight_scale), _scale_dtype(weight_scale), buffer(bias), buffer(y), flags, mode
         )
     )
 
