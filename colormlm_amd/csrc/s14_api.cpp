@@ -8,6 +8,7 @@
 // kernel launch on a stream; fences are hipEvents.
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -663,7 +664,7 @@ int prefill_workspace(s14_ctx *ctx) {
   const size_t o_w = take(sizeof(float) * T * kTopK);
   const size_t o_bits = take(sizeof(uint32_t) * kMaxExperts * kPrefillBitWords);
   const size_t o_items = take(sizeof(PrefillItem) * prefill_max_items(T));
-  const size_t o_stats = take(sizeof(uint32_t) * 4);
+  const size_t o_stats = take(sizeof(uint32_t) * kPrefillStats);
   const size_t o_pt = take(sizeof(uint32_t) * P);
   const size_t o_tp = take(sizeof(uint32_t) * T * kSlots);
   const size_t o_xq = take(size_t(T) * kHidden);
@@ -675,7 +676,7 @@ int prefill_workspace(s14_ctx *ctx) {
   const size_t o_hts = take(n_items * kHScaleBytes);
   const size_t o_down = take(sizeof(float) * size_t(P) * kHidden);
   const size_t o_pw = take(sizeof(float) * size_t(P));
-  const size_t o_hf = take(sizeof(float) * size_t(P) * kInter);
+  const size_t o_db = take(sizeof(uint16_t) * size_t(P) * kHidden);
   S14_HIP(hipSetDevice(ctx->device), "hipSetDevice");
   S14_HIP(hipMalloc(&ctx->prefill_base, off), "hipMalloc(prefill workspace)");
   // the token bitmaps start clear; every prefill's grouping step clears them again
@@ -702,7 +703,8 @@ int prefill_workspace(s14_ctx *ctx) {
   w.hts = b + o_hts;
   w.down = reinterpret_cast<float *>(b + o_down);
   w.pair_weight = reinterpret_cast<float *>(b + o_pw);
-  w.hf = reinterpret_cast<float *>(b + o_hf);
+  w.hb = reinterpret_cast<uint16_t *>(b + o_down);
+  w.down_b = reinterpret_cast<uint16_t *>(b + o_db);
   w.bytes = off;
   return S14_OK;
 }
@@ -837,9 +839,16 @@ extern "C" int s14_last_prefill_view(s14_ctx *ctx, s14_prefill_view *out) {
   if (!ctx->prefill_base || !ctx->prefill_tokens) return fail(S14_ERR_NOT_READY, "no prefill launched on this context");
   S14_HIP(hipSetDevice(ctx->device), "hipSetDevice");
   S14_HIP(hipDeviceSynchronize(), "hipDeviceSynchronize");
-  uint32_t st[4];
+  uint32_t st[s14::kPrefillStats];
   S14_HIP(hipMemcpy(st, ctx->pws.stats, sizeof(st), hipMemcpyDeviceToHost), "hipMemcpy(prefill stats)");
   const s14::PrefillWorkspace &w = ctx->pws;
+  if (st[4] == 1u) {  // the view's rows are f32; an official prefill keeps them as bf16
+    // (the count is garbage until a captured prefill has been replayed)
+    const uint32_t pairs = std::min(st[3], uint32_t(s14::kSlots) * s14::kMaxPrefillTokens);
+    const hipError_t e = s14::launch_prefill_down_f32(nullptr, w, pairs);
+    if (e != hipSuccess) return hip_fail(e, "prefill view launch");
+    S14_HIP(hipDeviceSynchronize(), "hipDeviceSynchronize");
+  }
   *out = s14_prefill_view{w.xq,
                           w.xs,
                           w.ht,

@@ -173,6 +173,7 @@ __global__ __launch_bounds__(1024) void k_prefill_group(PrefillArgs a, PrefillWo
       ws.stats[1] = distinct;
       ws.stats[2] = mx;
       ws.stats[3] = ic;  // number of pairs
+      ws.stats[4] = a.official ? 1u : 0u;
     }
   }
   __syncthreads();
@@ -450,13 +451,22 @@ __device__ __forceinline__ uint32_t h_scale_offset(uint32_t u, uint32_t b, uint3
   return (((u / kChunkSupers) * 2u + (col >> 4)) * 64u + (col & 15u) + 16u * b) * 4u + u % kChunkSupers;
 }
 
+// Two values that bf16_round returned, as stored bf16 (the low one first).
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+  return (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xffff0000u);
+}
+__device__ __forceinline__ float4 bf16x4_f32(uint2 v) {
+  return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                     __uint_as_float(v.y & 0xffff0000u));
+}
+
 // Phase 1: one wavefront per (32-row tile of w1/w3, work item of <= 32
 // pairs of one expert), NH column halves.  K = 4096 in 16 chunks; weights
 // kRing - 1 chunks ahead in LDS, activations kRing chunks ahead in VGPRs.
 // Then h = swiglu(g, u), requantised per token over the tile's 32 rows (one
 // E8M0 group of phase 2's K) and stored into the item's phase-2 tile.
 // kOfficial: h = bf16(swiglu(bf16(g), bf16(u)) * w), w the pair's route
-// weight (1 for the shared expert) (executor.py:717-731), stored in f32 for
+// weight (1 for the shared expert) (executor.py:717-731), stored as bf16 for
 // k_requant_h128 (its group of 128 rows spans four of these workgroups).
 template <bool kOfficial, int NH>
 __device__ __forceinline__ void prefill_up_item(const PrefillArgs &a, const PrefillWorkspace &ws,
@@ -573,7 +583,7 @@ __device__ __forceinline__ void prefill_up_item(const PrefillArgs &a, const Pref
       if (col >= it.count) continue;
       const uint32_t pair = it.first + col;
       const float w = ws.pair_weight[pair];
-      float *dst = ws.hf + size_t(pair) * kInter + rt * 32u;
+      uint16_t *dst = ws.hb + size_t(pair) * kInter + rt * 32u;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         float o[4];
@@ -581,7 +591,7 @@ __device__ __forceinline__ void prefill_up_item(const PrefillArgs &a, const Pref
         for (int v = 0; v < 4; ++v)
           o[v] = bf16_round(
               __fmul_rn(swiglu_exact(bf16_round(acc[4 * h + i][v]), bf16_round(acc[4 * h + 2 + i][v]), exptab), w));
-        *reinterpret_cast<float4 *>(dst + 16u * uint32_t(i) + 4u * q) = make_float4(o[0], o[1], o[2], o[3]);
+        *reinterpret_cast<uint2 *>(dst + 16u * uint32_t(i) + 4u * q) = make_uint2(bf16_pair(o[0], o[1]), bf16_pair(o[2], o[3]));
       }
     }
     return;
@@ -638,7 +648,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 // h columns into the item's phase-2 tile and scales, in the layout
 // k_prefill_up's epilogue writes otherwise (tile rt holds rows 32 rt .. +31,
 // half rt % 2 of K step rt / 2).  Eight lanes per (item, column, 128 rows),
-// each lane 16 rows (64 contiguous bytes in, one 16-byte piece out); the
+// each lane 16 rows (32 contiguous bytes in, one 16-byte piece out); the
 // group's maximum by xor shuffles within the eight.
 constexpr uint32_t kHGroups128 = kInter / 128;
 __global__ __launch_bounds__(256) void k_requant_h128(PrefillWorkspace ws) {
@@ -649,13 +659,13 @@ __global__ __launch_bounds__(256) void k_requant_h128(PrefillWorkspace ws) {
   const uint32_t col = (grp / kHGroups128) % kItemTokens, m = grp % kHGroups128;
   const PrefillItem it = ws.items[item];
   if (col >= it.count) return;  // phase 2 never reads absent columns
-  const float4 *src =
-      reinterpret_cast<const float4 *>(ws.hf + size_t(it.first + col) * kInter + 128u * m + 16u * j);
-  float4 q[4];
+  const uint4 *src = reinterpret_cast<const uint4 *>(ws.hb + size_t(it.first + col) * kInter + 128u * m + 16u * j);
+  const uint4 s0 = src[0], s1 = src[1];
+  const float4 q[4] = {bf16x4_f32(make_uint2(s0.x, s0.y)), bf16x4_f32(make_uint2(s0.z, s0.w)),
+                       bf16x4_f32(make_uint2(s1.x, s1.y)), bf16x4_f32(make_uint2(s1.z, s1.w))};
   float amax = 0.0f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    q[i] = src[i];
     amax = fabsf(q[i].x) > amax ? fabsf(q[i].x) : amax;
     amax = fabsf(q[i].y) > amax ? fabsf(q[i].y) : amax;
     amax = fabsf(q[i].z) > amax ? fabsf(q[i].z) : amax;
@@ -779,13 +789,15 @@ __device__ __forceinline__ void prefill_down_item(const PrefillArgs &a, const Pr
   for (int h = 0; h < NH; ++h) {
     const uint32_t col = 16u * uint32_t(h) + c16;
     if (col >= it.count) continue;
-    float *dst = ws.down + size_t(it.first + col) * kHidden + rt * kDnRows + 4u * q;
+    const size_t at = size_t(it.first + col) * kHidden + rt * kDnRows + 4u * q;
 #pragma unroll
     for (int tl = 0; tl < NT; ++tl) {
       const v4f v = d[NT * h + tl];
-      float4 o = make_float4(v[0], v[1], v[2], v[3]);
-      if constexpr (kOfficial) o = make_float4(bf16_round(o.x), bf16_round(o.y), bf16_round(o.z), bf16_round(o.w));
-      *reinterpret_cast<float4 *>(dst + 16u * uint32_t(tl)) = o;
+      if constexpr (kOfficial)
+        *reinterpret_cast<uint2 *>(ws.down_b + at + 16u * uint32_t(tl)) =
+            make_uint2(bf16_pair(bf16_round(v[0]), bf16_round(v[1])), bf16_pair(bf16_round(v[2]), bf16_round(v[3])));
+      else
+        *reinterpret_cast<float4 *>(ws.down + at + 16u * uint32_t(tl)) = make_float4(v[0], v[1], v[2], v[3]);
     }
   }
 }
@@ -824,9 +836,15 @@ __global__ __launch_bounds__(256) void k_prefill_combine(PrefillArgs a, PrefillW
   for (uint32_t s = 0; s < uint32_t(kTopK); ++s) wt[s] = s < k ? ws.weights[t * kTopK + s] : 0.0f;
   float4 d[kSlots];
 #pragma unroll
-  for (uint32_t s = 0; s < uint32_t(kSlots); ++s)
-    d[s] = s <= k ? *reinterpret_cast<const float4 *>(ws.down + size_t(pr[s]) * kHidden + r)
-                  : make_float4(0.f, 0.f, 0.f, 0.f);
+  for (uint32_t s = 0; s < uint32_t(kSlots); ++s) {
+    const size_t at = size_t(pr[s]) * kHidden + r;
+    if (s > k)
+      d[s] = make_float4(0.f, 0.f, 0.f, 0.f);
+    else if constexpr (kOfficial)
+      d[s] = bf16x4_f32(*reinterpret_cast<const uint2 *>(ws.down_b + at));
+    else
+      d[s] = *reinterpret_cast<const float4 *>(ws.down + at);
+  }
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (uint32_t s = 0; s < uint32_t(kSlots); ++s) {
@@ -847,7 +865,17 @@ __global__ __launch_bounds__(256) void k_prefill_combine(PrefillArgs a, PrefillW
   *reinterpret_cast<float4 *>(a.y + size_t(t) * kHidden + r) = acc;
 }
 
+__global__ __launch_bounds__(256) void k_prefill_down_f32(PrefillWorkspace ws) {
+  const size_t i = 4u * (size_t(blockIdx.x) * 256u + threadIdx.x);  // whole workgroups: kHidden / 1024 a pair
+  *reinterpret_cast<float4 *>(ws.down + i) = bf16x4_f32(*reinterpret_cast<const uint2 *>(ws.down_b + i));
+}
+
 }  // namespace
+
+hipError_t launch_prefill_down_f32(hipStream_t s, const PrefillWorkspace &ws, uint32_t pairs) {
+  if (pairs) k_prefill_down_f32<<<pairs * (kHidden / 1024), 256, 0, s>>>(ws);
+  return hipGetLastError();
+}
 
 hipError_t launch_prefill(hipStream_t s, const PrefillArgs &a, const PrefillWorkspace &ws) {
   const uint32_t T = a.tokens;

@@ -56,6 +56,8 @@ struct PrefillArgs {
   int official;      // 1: the official expert semantics (S14_MODE_OFFICIAL)
 };
 
+constexpr uint32_t kPrefillStats = 5;  // words of PrefillWorkspace::stats
+
 // Device workspace for up to kMaxPrefillTokens tokens (one allocation per
 // context, made on the first prefill call).
 struct PrefillWorkspace {
@@ -65,7 +67,7 @@ struct PrefillWorkspace {
   float *weights;         // [T][kTopK]
   uint32_t *token_bits;   // [256][kPrefillBitWords]
   PrefillItem *items;     // [prefill_max_items]
-  uint32_t *stats;        // {items, distinct routed experts, max tokens per expert, pairs}
+  uint32_t *stats;        // {items, distinct routed experts, max tokens per expert, pairs, official}
   uint32_t *pair_token;   // [7T]
   uint32_t *token_pair;   // [T][kSlots]
   uint8_t *xq;            // [T][4096] e4m3
@@ -76,10 +78,16 @@ struct PrefillWorkspace {
   uint8_t *hts;           // [items][kHScaleBytes]
   float *down;            // [7T][4096]
   float *pair_weight;     // [7T]: each pair's route weight (1 for the shared expert)
-  float *hf;              // [7T][2048]: official mode's h (bf16 values) before its group-128 requant
+  // Official mode rounds h and the down rows to bf16 and stores them in that
+  // type, the same values in half the bytes (both f32: 1023 us at 1024 tokens;
+  // as bf16: 1002):
+  uint16_t *hb;           // [7T][2048] h before its group-128 requant, in down's memory
+  uint16_t *down_b;       // [7T][4096] down rows (down holds them in f32 only for a view)
   size_t bytes;
 };
 
 hipError_t launch_prefill(hipStream_t s, const PrefillArgs &a, const PrefillWorkspace &ws);
+// down = down_b, for a view of an official prefill of `pairs` pairs.
+hipError_t launch_prefill_down_f32(hipStream_t s, const PrefillWorkspace &ws, uint32_t pairs);
 
 }  // namespace s14

@@ -975,6 +975,38 @@ def test_prefill_official(ctx, oracle, bank, prefill_router, tokens):
     assert_bit_exact(y3, y[pick], f"official rows {pick} vs a {len(pick)}-token run")
 
 
+@pytest.mark.parametrize("tokens", [1, 33])
+def test_prefill_official_rows_across_modes(ctx, bank, prefill_router, tokens):
+    """Official prefills keep their h and down rows as bf16 in memory that a
+    default prefill's f32 rows use too.  An official prefill captured in a
+    graph, replayed with a default prefill on the same context in between:
+    every replay's view shows the eager run's rows (bf16 values) and output,
+    and the default prefill's rows stay f32."""
+    say(f"official prefill T={tokens} in a graph, default prefills between the replays")
+    xs = synth.prefill_tokens(seed=4, tokens=tokens)
+    want_y, _, _ = _run_prefill_official(ctx, bank, prefill_router, xs)
+    want = s14.last_prefill_view(ctx)["down"]
+    assert_bit_exact(want, _bf16(want), "down rows are bf16 values")
+    y_def, _, _ = _run_prefill(ctx, bank, prefill_router, xs)
+    want_def = s14.last_prefill_view(ctx)["down"]
+    assert not np.array_equal(want_def, _bf16(want_def)), "default rows stay f32"
+    x, y = dev(xs), torch.empty((tokens, HIDDEN), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        s14.moe_prefill(ctx, tokens, prefill_router["router"], bank["table"], bank["pages"][256], x, y,
+                        mode=s14.OFFICIAL)
+    for i in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert_bit_exact(s14.last_prefill_view(ctx)["down"], want, f"replay {i}: down rows")
+        assert_bit_exact(host(y), want_y, f"replay {i}: output")
+        got, _, _ = _run_prefill(ctx, bank, prefill_router, xs)
+        assert_bit_exact(got, y_def, f"default prefill after replay {i}")
+        assert_bit_exact(s14.last_prefill_view(ctx)["down"], want_def, f"default rows after replay {i}")
+    del g
+
+
 @pytest.mark.parametrize("tokens", [1, 5, 1024])
 def test_prefill_ragged_and_max_tokens(ctx, oracle, bank, prefill_router, tokens):
     """1 and 5 tokens (partial MFMA column tiles) and the 1024-token maximum:
