@@ -20,3 +20,16 @@ extern "C" void lin_limits(uint64_t *part_bytes, uint32_t *counters, uint32_t *s
   *stage_bytes = s14::kLinStageBytes;
   *tile = s14::kLinTile;
 }
+
+extern "C" void lin_gemm(uint32_t m, uint32_t n, uint32_t groups, uint32_t *tokens, uint32_t *splits) {
+  const s14::LinGemmPlan p = s14::lin_gemm_plan(m, n, groups);
+  *tokens = p.tokens;
+  *splits = p.splits;
+}
+
+extern "C" uint32_t lin_exact(uint32_t m, uint32_t n, uint32_t groups, uint32_t *tokens, uint32_t *waves) {
+  const s14::LinExactPlan p = s14::lin_exact_plan(m, n, groups);
+  *tokens = p.tokens;
+  *waves = p.waves;
+  return s14::lin_exact_first(m, n, groups);
+}

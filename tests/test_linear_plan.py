@@ -104,3 +104,28 @@ def test_fast_plan_hands_unplannable_shapes_to_exact(plan_lib):
     for m in (1, 2, 31, 32, 33, 300, 1024):
         for n, k in ((65536, 16384), (100, 131072), (131072, 512), (4096, 65536)):
             check(plan_lib, m, n, k)
+
+
+@pytest.mark.parametrize("n,k", [*SHAPES.values(), (1, 512), (65, 12800), (131072, 512), (100, 131072)])
+def test_prompt_tile_and_exact_mfma_plans(plan_lib, n, k):
+    """The FAST prompt tiles: every K split holds a group and the partial sums
+    fit the workspace.  The EXACT f32-MFMA plan: one of the kernels that
+    launch_exact_plan has, for one launch and for both parts of two (the first
+    of whole 32-token blocks)."""
+    groups = k // 128
+    a, b = C.c_uint32(), C.c_uint32()
+    kinds = {(4, 4), (4, 16), (8, 4), (8, 8), (16, 4), (16, 8), (32, 4)}
+    for m in [*range(1, 400), 511, 512, 513, 1023, 1024, 5000]:
+        plan_lib.lin_gemm(C.c_uint32(m), C.c_uint32(n), C.c_uint32(groups), C.byref(a), C.byref(b))
+        tokens, splits = a.value, b.value
+        assert tokens in (32, 64) and splits >= 1
+        if splits > 1:
+            per = -(-groups // splits)
+            assert per >= 4 and (splits - 1) * per < groups, (m, splits)
+            assert splits * m * n * 4 <= 32 << 20, (m, splits)
+        first = plan_lib.lin_exact(C.c_uint32(m), C.c_uint32(n), C.c_uint32(groups), C.byref(a), C.byref(b))
+        assert (a.value, b.value) in kinds
+        assert first == m or (0 < first < m and first % 32 == 0), (m, first)
+        for part in {first, m - first} - {0}:
+            plan_lib.lin_exact(C.c_uint32(part), C.c_uint32(n), C.c_uint32(groups), C.byref(a), C.byref(b))
+            assert (a.value, b.value) in kinds
