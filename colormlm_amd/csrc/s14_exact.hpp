@@ -1160,6 +1160,79 @@ __device__ __forceinline__ CodeWindow requant128_block(float *v, int n, int *red
   return mx_window(lo, hi);
 }
 
+// Scale code of a group whose largest magnitude has the bits `amax` (finite):
+// requant_code without its division.  448 = 1.75 * 2^8: the quotient's
+// ceil(log2) steps up where the mantissa passes 1.75 (0x600000), and the
+// rounding of the quotient never crosses a power of two.
+__device__ __forceinline__ uint32_t requant_code_bits(uint32_t amax) {
+  return ((max(amax, 0x38d1b717u) + 0x1fffffu) >> 23) - 8u;  // 0x38d1b717: 1e-4
+}
+// act_quant (groups of 128) of the vectors that stage_load_wave left in
+// registers, and their decode windows.  Load `it` gives lanes 0-31 one group
+// and lanes 32-63 the next, four values a lane: the group's maximum by DPP
+// steps and a permlane swap, the codes by the hardware's e4m3 conversions
+// (round to nearest even; nothing reaches past 448 here).  The window comes
+// from the scales: a nonzero result lies in [2^-9, 448] times its group's.
+// Returns the vectors left as they are (bit s): those with a magnitude past
+// 2^100, an infinity or a NaN, which requant128_staged takes once they are in
+// LDS.
+template <int N, int S>
+__device__ __forceinline__ uint32_t requant128_regs(StageRegs<N, S> &r, CodeWindow (&win)[2]) {
+  constexpr int IT = N / 256;
+  uint32_t slow = 0;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    uint32_t am[IT], top = 0;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const float4 v = r.v[s][it];
+      uint32_t m = max(max(__float_as_uint(v.x) & 0x7fffffffu, __float_as_uint(v.y) & 0x7fffffffu),
+                       max(__float_as_uint(v.z) & 0x7fffffffu, __float_as_uint(v.w) & 0x7fffffffu));
+      m = max(m, uint32_t(dpp_i<0xb1>(0, int(m))));   // quad_perm [1,0,3,2]
+      m = max(m, uint32_t(dpp_i<0x4e>(0, int(m))));   // quad_perm [2,3,0,1]
+      m = max(m, uint32_t(dpp_i<0x141>(0, int(m))));  // row_half_mirror
+      m = max(m, uint32_t(dpp_i<0x140>(0, int(m))));  // row_mirror
+      const auto sw = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+      am[it] = max(sw[0], sw[1]);
+      top = max(top, am[it]);
+    }
+    if (__builtin_amdgcn_ballot_w64(top > 0x71800000u) == 0ull) {
+      int lo = 255, hi = 0;
+#pragma unroll
+      for (int it = 0; it < IT; ++it) {
+        const uint32_t code = requant_code_bits(am[it]);
+        const float inv = __uint_as_float((254u - code) << 23), sc = __uint_as_float(code << 23);
+        float4 &v = r.v[s][it];
+        uint32_t q = uint32_t(__builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(v.x, inv), __fmul_rn(v.y, inv), 0, false));
+        q = uint32_t(__builtin_amdgcn_cvt_pk_fp8_f32(__fmul_rn(v.z, inv), __fmul_rn(v.w, inv), int(q), true));
+        const v2f a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(q, sc, false);
+        const v2f b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(q, sc, true);
+        v = make_float4(a.x, a.y, b.x, b.y);
+        lo = min(lo, int(code) - 9);
+        hi = max(hi, int(code) + 8);
+      }
+      win[s] = mx_window(wave_min_i(lo), wave_max_i(hi));
+    } else {
+      slow |= 1u << s;
+    }
+  }
+  return slow;
+}
+// What requant128_regs left, after stage_store_wave: by the bitwise conversion,
+// the calling wavefront's own copies.
+template <int N, int S>
+__device__ __forceinline__ void requant128_staged(float *const (&dst)[S], uint32_t slow, CodeWindow (&win)[2]) {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    if (!(slow >> s & 1u)) continue;
+    int lo = 255, hi = 0;
+    requant128_groups(dst[s], N / 128, 0, 1, lo, hi);
+    win[s] = mx_window(wave_min_i(lo), wave_max_i(hi));
+  }
+}
+
 // Groups per register batch in the fused exact kernels.  Larger batches hide
 // more load latency but inline a longer straight-line body; on the box 8
 // beat 16 by 10 % per layer (instruction supply) and 4 (batch overhead).

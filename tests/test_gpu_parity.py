@@ -1322,6 +1322,21 @@ def test_official_chain_weight_before_w2(ctx, oracle, bank):
     assert_bit_exact(host(y), want, "official chain")
 
 
+@pytest.mark.parametrize("w", [0.0, 1e-38, 3e-6, 1e30, 1e35])
+def test_official_chain_h_quant_range(ctx, oracle, bank, w):
+    """h's act_quant inside phase 2 over the range that the route weight can
+    give it: all zero, groups at the quant's 1e-4 floor (every value rounding
+    to zero or to the smallest steps), and groups on both sides of 2^100, where
+    it leaves the hardware's conversions; ordinary weights are the tests
+    around this one."""
+    say(f"official chain, route weight {w}")
+    cfg = synth.config0(seed=6)
+    want = oracle.moe_layer_official(cfg["x"], [cfg["page"]], np.array([w], np.float32), None)
+    y = torch.empty(HIDDEN, dtype=torch.float32, device="cuda")
+    s14.expert_chain(ctx, dev(cfg["page"]), dev(cfg["x"]), w, y, mode=s14.OFFICIAL)
+    assert_bit_exact(host(y), want, f"official chain, weight {w}")
+
+
 @pytest.mark.parametrize("score_fn,scale,tokens", [(N.S14_SCORE_SIGMOID, 1.0, 8),
                                                    (N.S14_SCORE_SQRT_SOFTPLUS, 1.5, 3),
                                                    (N.S14_SCORE_SIGMOID, 1.0, 2)])
