@@ -1160,13 +1160,6 @@ __device__ __forceinline__ CodeWindow requant128_block(float *v, int n, int *red
   return mx_window(lo, hi);
 }
 
-// Scale code of a group whose largest magnitude has the bits `amax` (finite):
-// requant_code without its division.  448 = 1.75 * 2^8: the quotient's
-// ceil(log2) steps up where the mantissa passes 1.75 (0x600000), and the
-// rounding of the quotient never crosses a power of two.
-__device__ __forceinline__ uint32_t requant_code_bits(uint32_t amax) {
-  return ((max(amax, 0x38d1b717u) + 0x1fffffu) >> 23) - 8u;  // 0x38d1b717: 1e-4
-}
 // act_quant (groups of 128) of the vectors that stage_load_wave left in
 // registers, and their decode windows.  Load `it` gives lanes 0-31 one group
 // and lanes 32-63 the next, four values a lane: the group's maximum by DPP

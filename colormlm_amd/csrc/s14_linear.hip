@@ -79,12 +79,9 @@ __global__ __launch_bounds__(256) void k_act_quant(uint32_t n_quads, const float
     const float o = __shfl_xor(amax, int(d));
     amax = o > amax ? o : amax;
   }
-  const uint32_t code = requant_code(amax);
-  const float inv = __uint_as_float((254u - code) << 23);
-  reinterpret_cast<uint32_t *>(Q)[i] =
-      s14x::e4m3_rne_sat(__fmul_rn(v.x, inv)) | (s14x::e4m3_rne_sat(__fmul_rn(v.y, inv)) << 8) |
-      (s14x::e4m3_rne_sat(__fmul_rn(v.z, inv)) << 16) | (s14x::e4m3_rne_sat(__fmul_rn(v.w, inv)) << 24);
-  if (i % kLanes == 0) S[i / kLanes] = uint8_t(code);
+  const GroupQuant gq(amax);
+  reinterpret_cast<uint32_t *>(Q)[i] = gq.word(v.x, v.y, v.z, v.w);
+  if (i % kLanes == 0) S[i / kLanes] = uint8_t(gq.code);
 }
 
 // One thread per group: x not 16-byte or q not 4-byte aligned.

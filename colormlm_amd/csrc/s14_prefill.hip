@@ -39,8 +39,6 @@ constexpr uint32_t kQGroup = 32;  // requant group (k values per E8M0 scale)
 // requant (bit-identical to the oracle's s14o_requant_e4m3)
 // ---------------------------------------------------------------------------
 
-using s14x::e4m3_rne_sat;  // s14_e4m3.h: straight-line, checked against the oracle on the CPU
-
 // The activation requant X [T, 4096] f32 -> Q [T, 4096] e4m3 + S [T, 128]
 // E8M0 (requant_x_group) runs in extra workgroups of the router's launch
 // (launch_router_scores), beside the scoring it does not depend on.
@@ -614,19 +612,16 @@ __device__ __forceinline__ void prefill_up_item(const PrefillArgs &a, const Pref
       const float other = __shfl_xor(amax, m);
       amax = other > amax ? other : amax;
     }
-    const uint32_t code = requant_code(amax);
-    const float inv = __uint_as_float((254u - code) << 23);
+    const GroupQuant gq(amax);
     const uint32_t col = 16u * uint32_t(h) + c16;
     if (col >= it.count) continue;  // phase 2 never reads absent columns
 #pragma unroll
     for (int i = 0; i < 2; ++i) {  // rows 16 i + 4 q .. +3: plane i, bytes 4 q .. 4 q + 3
-      uint32_t word = 0;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) word |= e4m3_rne_sat(__fmul_rn(hv[4 * i + v], inv)) << (8 * v);
+      const uint32_t word = gq.word(hv[4 * i], hv[4 * i + 1], hv[4 * i + 2], hv[4 * i + 3]);
       *reinterpret_cast<uint32_t *>(ws.ht + size_t(item) * kHTileBytes + h_tile_offset(u2, b2, uint32_t(i), col) +
                                     4u * q) = word;
     }
-    if (q == 0) ws.hts[size_t(item) * kHScaleBytes + h_scale_offset(u2, b2, col)] = uint8_t(code);
+    if (q == 0) ws.hts[size_t(item) * kHScaleBytes + h_scale_offset(u2, b2, col)] = uint8_t(gq.code);
   }
 }
 
@@ -676,17 +671,14 @@ __global__ __launch_bounds__(256) void k_requant_h128(PrefillWorkspace ws) {
     const float o = __shfl_xor(amax, d);
     amax = o > amax ? o : amax;
   }
-  const uint32_t code = requant_code(amax);
-  const float inv = __uint_as_float((254u - code) << 23);
+  const GroupQuant gq(amax);
   uint32_t w[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    w[i] = e4m3_rne_sat(__fmul_rn(q[i].x, inv)) | (e4m3_rne_sat(__fmul_rn(q[i].y, inv)) << 8) |
-           (e4m3_rne_sat(__fmul_rn(q[i].z, inv)) << 16) | (e4m3_rne_sat(__fmul_rn(q[i].w, inv)) << 24);
+  for (int i = 0; i < 4; ++i) w[i] = gq.word(q[i].x, q[i].y, q[i].z, q[i].w);
   // group m is phase 2's super-step m: piece j is plane j % 2 of block j / 2
   *reinterpret_cast<uint4 *>(ws.ht + size_t(item) * kHTileBytes + h_tile_offset(m, j >> 1, j & 1u, col)) =
       make_uint4(w[0], w[1], w[2], w[3]);
-  if ((j & 1u) == 0) ws.hts[size_t(item) * kHScaleBytes + h_scale_offset(m, j >> 1, col)] = uint8_t(code);
+  if ((j & 1u) == 0) ws.hts[size_t(item) * kHScaleBytes + h_scale_offset(m, j >> 1, col)] = uint8_t(gq.code);
 }
 
 // Phase 2: one wavefront per (64-row tile of w2, work item): down rows of

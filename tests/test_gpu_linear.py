@@ -125,6 +125,30 @@ def test_act_quant_alignment_and_odd_sizes(ctx, oracle, rows, k):
         assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]), group
 
 
+@pytest.mark.parametrize("group", [32, 64, 128])
+def test_act_quant_conversion_range(ctx, oracle, group):
+    """Group maxima on both sides of 2^100, where the codes leave the
+    hardware's conversion, up to the largest f32 and down to zero, of and just
+    past 448 times a power of two (where the scale steps), with NaNs beside
+    them: codes and scales equal the oracle's."""
+    say(f"act quant conversion range group={group}")
+    rng = np.random.default_rng(group)
+    f = np.float32
+    tops = [f(2.0**100), np.nextafter(f(2.0**100), f(np.inf)), f(3.4028235e38), f(1e-4), f(9e-5), f(1e-40), f(0.0)]
+    for e in (-20, 0, 60, 95):
+        t = f(448.0 * 2.0**e)
+        tops += [t, np.nextafter(t, f(np.inf)), np.nextafter(t, f(0.0))]
+    x = (rng.uniform(-1, 1, (len(tops), 128)) * np.exp2(rng.integers(-18, 1, (len(tops), 128)))).astype(f)
+    x *= np.array(tops, f)[:, None]
+    x[:, ::group] = np.array(tops, f)[:, None]
+    x[::2, 5], x[1::3, 7] = np.nan, -np.nan
+    q = torch.empty(x.shape, dtype=torch.uint8, device="cuda")
+    s = torch.empty((x.shape[0], 128 // group), dtype=torch.uint8, device="cuda")
+    s14.act_quant_e4m3(ctx, dev(x), q, s, group=group)
+    want = oracle.requant_e4m3(x, group=group)
+    assert np.array_equal(host(s), want[1]) and np.array_equal(host(q), want[0])
+
+
 @pytest.mark.parametrize("m", [1, 4])
 @pytest.mark.parametrize("name", list(SHAPES))
 def test_fp8_linear_projection_shapes(ctx, oracle, name, m):
