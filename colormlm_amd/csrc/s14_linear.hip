@@ -1500,7 +1500,8 @@ hipError_t launch_fp8_linear(hipStream_t s, const LinearArgs &a, int mode, const
   // past 4,096 stay on the tiles below (wo_b m = 4: 21.5 us against 24.1:
   // 64-row workgroups leave most CUs idle there)
   if (vec && a.k % kLinGroup == 0u && !a.x_scale_f32 && !a.w_scale_f32 && (a.m > 4u || a.k <= 4096u) &&
-      uint64_t(a.n + kXmRows - 1) * a.k <= 0xFFFFFFFFull) {
+      uint64_t(a.n + kXmRows - 1) * a.k <= 0xFFFFFFFFull &&
+      !(size_t(a.groups) * a.n * sizeof(float) <= kLinPartBytes && lin_exact_tiles(a.m, a.n, a.groups))) {
     const uint32_t first = lin_exact_first(a.m, a.n, a.groups);
     LinearArgs c = a;
     c.m = first;

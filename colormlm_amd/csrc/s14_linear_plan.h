@@ -149,4 +149,18 @@ inline uint32_t lin_exact_first(uint32_t m, uint32_t n, uint32_t G) {
   return first;
 }
 
+// Is k_linear_tile with k_linear_sum estimated faster than the f32 MFMA
+// kernel?  Few rows and tokens leave that one a few workgroups whose
+// wavefronts take several groups each, where the tiles have a wavefront per
+// group: their time goes by rounds of 1,024 wavefronts (graph replays, us,
+// tiles / f32 MFMA: [512, 4096] 8 tokens 10.0 / 11.9, 32 tokens 10.8 / 12.0, 64
+// tokens 15.5 / 12.2; [2048, 4096] 8 tokens 10.7 / 12.1, 12 tokens 15.3 / 12.1;
+// [1024, 8192] 16 tokens 17.1 / 21.5, 32 tokens 26.9 / 21.7; [512, 2048] 2 tokens
+// 5.4 / 6.9, 5 tokens 9.1 / 7.1).  The MFMA estimate lacks the launch.
+inline bool lin_exact_tiles(uint32_t m, uint32_t n, uint32_t G) {
+  const uint64_t waves = (uint64_t(n) + 63u) / 64u * G * ((uint64_t(m) + 7u) / 8u);
+  const uint64_t first = m <= 2u ? 5600u : m <= 4u ? 6800u : 9500u, more = m <= 2u ? 2200u : m <= 4u ? 3000u : 5200u;
+  return first + (waves + 1023u) / 1024u * more - more < lin_exact_plan(m, n, G).ns + 2000u;
+}
+
 }  // namespace s14
