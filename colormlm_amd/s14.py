@@ -60,7 +60,24 @@ def _scale_dtype(t) -> int:
     return code
 
 
-_TORCH_CUDA = []  # [torch] once torch with a visible GPU is found, [None] if not
+_CURRENT_STREAM = []  # [function returning torch's current stream], [None] without torch or a GPU
+
+
+def _current_stream():
+    """torch.cuda.current_stream().cuda_stream, without the object where this
+    torch has the two raw calls (they initialise its GPU state the same way, and
+    fail the same way); None without torch or a GPU."""
+    try:
+        import torch
+
+        if not torch.cuda.is_available():
+            return None
+    except Exception:  # pragma: no cover - torch is optional for the ABI
+        return None
+    raw, device = (getattr(torch._C, f, None) for f in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+    if raw is None or device is None:
+        return lambda: torch.cuda.current_stream().cuda_stream
+    return lambda: raw(device())
 
 
 def _stream(stream):
@@ -69,19 +86,10 @@ def _stream(stream):
     null stream."""
     if stream is not None:
         return stream
-    if not _TORCH_CUDA:
-        try:
-            import torch
-
-            if torch.cuda.is_available():
-                torch.cuda.init()  # before the raw stream is asked for below
-            _TORCH_CUDA.append(torch if torch.cuda.is_available() else None)
-        except Exception:  # pragma: no cover - torch is optional for the ABI
-            _TORCH_CUDA.append(None)
-    torch = _TORCH_CUDA[0]
-    if torch is None:
-        return None
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())  # current_stream().cuda_stream without the object
+    if not _CURRENT_STREAM:
+        _CURRENT_STREAM.append(_current_stream())
+    current = _CURRENT_STREAM[0]
+    return current() if current is not None else None
 
 
 class Context:
