@@ -29,7 +29,7 @@ struct s14_ctx {
   int device = 0;
   hipStream_t compute = nullptr;
   hipStream_t copy = nullptr;
-  s14::BlockFork fork{};  // side stream and events of EXACT blocks
+  s14::BlockFork fork{};  // side stream and events of blocks
   void *ws_base = nullptr;
   void *prefill_base = nullptr;  // prefill workspace, made on the first prefill call
   void *lin_base = nullptr;      // fp8_linear FAST split-K workspace, made on the first FAST call
@@ -477,6 +477,34 @@ int block_route_validate(uint32_t tokens, const s14_router *router, const uint64
   return S14_OK;
 }
 
+// Does a block of `tokens` run its pairs as two halves on two streams?  The
+// SIMDs that one half's phase-1 tail leaves idle (two equal wavefronts resident
+// a SIMD, of 2.2 at 5 tokens, 3.1 at 7 and 3.5 at 8) take the other half's work.  Launched eagerly the fork and the join cost up
+// to 27 us of event latency; a captured graph's branches do not.  us a block,
+// one stream / two, MXFP4 shared page (FP8 in brackets):
+//   graph, EXACT: 2 tokens 60.6 / 87.6, 4 101.9 / 103.7 (130.4 / 132.5), 5 134.7 / 133.7
+//     (160.2 / 157.2), 6 138.5 / 139.9 (163.8 / 166.4), 7 167.6 / 156.3 (193.3 / 183.0),
+//     8 174.0 / 164.4 (196.9 / 192.1); 3 within 0.7 of each other
+//   graph, official: 4 97.1 / 98.3, 5 123.6 / 125.1, 6 127.9 / 133.3 (153.1 / 162.0),
+//     7 153.5 / 147.4 (182.8 / 179.5), 8 161.4 / 158.8 (186.5 / 192.9)
+//   eager, EXACT: 5 134.4 / 140.7, 6 138.3 / 147.4, 7 163.6 / 159.4, 8 168.6 / 165.8;
+//   eager, official: 7 149.6 / 150.3, 8 156.2 / 159.8
+static bool block_forks(uint32_t tokens, bool official, int shared_format, bool graph) {
+  if (!graph) return !official && tokens >= 7;
+  if (tokens == 8) return !official || shared_format == S14_PAGE_MXFP4;
+  return tokens == 7 || (tokens == 5 && !official);
+}
+// Is `st` being captured into a graph?  (The null stream cannot be.)
+static bool captured(hipStream_t st) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (!st) return false;
+  if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+    (void)hipGetLastError();  // not this launch's error
+    return false;
+  }
+  return status == hipStreamCaptureStatusActive;
+}
+
 int block_route_launch(hipStream_t st, const Workspace &ws, uint32_t tokens, const s14_router *router,
                        const uint64_t *expert_pages_dev, const uint8_t *shared_page, int shared_format,
                        const float *x, float *y, uint16_t *ids_out, float *weights_out, int mode,
@@ -506,15 +534,10 @@ int block_route_launch(hipStream_t st, const Workspace &ws, uint32_t tokens, con
   if (e != hipSuccess) return hip_fail(e, "router launch");
   if (tokens > 1 && (mode == S14_MODE_EXACT || official)) {
     // blocks: one row per lane (enough (token, expert) chains to fill the
-    // GPU).  With a side stream the pairs can run as two halves, one per
-    // stream, so that the SIMDs one half's phase-1 tail leaves idle (3.5 equal
-    // wavefronts per SIMD, two resident at a time) take the other half's
-    // work.  The fork and the join cost about 18 us of event latency, so it
-    // pays only for the longest blocks (us, one stream against two: EXACT
-    // T = 2 61.5 / 95.8, 4 98.0 / 108.4, 6 135.2 / 143.3, 7 163.3 / 160.3, 8 170.9 /
-    // 168.1; official T = 8 158.5 / 161.9).  An even split measured best; three
-    // or four streams were slower.  Stage events time the first half.
-    if (official || tokens < 7) fork = nullptr;
+    // GPU); with a side stream the pairs can run as two halves, one per stream
+    // (block_forks).  An even split measured best; three or four streams were
+    // slower.  Stage events time the first half.
+    if (fork && !block_forks(tokens, official, shared_format, captured(st))) fork = nullptr;
     const uint32_t na = fork ? n_pairs / 2 : n_pairs, nb = n_pairs - na;
     if (fork) {
       if ((e = hipEventRecord(fork->fork, st)) != hipSuccess) return hip_fail(e, "hipEventRecord(fork)");

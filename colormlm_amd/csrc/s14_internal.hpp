@@ -17,14 +17,14 @@ namespace s14 {
 int block_route_validate(uint32_t tokens, const s14_router *router, const uint64_t *expert_pages_dev,
                          const uint8_t *shared_page, int shared_format, const float *x, float *y, int mode);
 // A second stream and two events (all on the context's device) over which
-// an EXACT block runs half of its pairs beside the caller's stream.
+// a block runs half of its pairs beside the caller's stream (block_forks).
 struct BlockFork {
   hipStream_t side;
   hipEvent_t fork, join;
 };
 // Route -> phase 1 -> phase 2 of a routed layer/block on `st` with workspace
 // `ws` (arguments already validated); ev: per-stage timing events or NULL;
-// fork: the side stream for EXACT blocks, or NULL to run everything on `st`.
+// fork: a side stream for blocks, or NULL to run everything on `st`.
 int block_route_launch(hipStream_t st, const Workspace &ws, uint32_t tokens, const s14_router *router,
                        const uint64_t *expert_pages_dev, const uint8_t *shared_page, int shared_format,
                        const float *x, float *y, uint16_t *ids_out, float *weights_out, int mode,

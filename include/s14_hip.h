@@ -277,7 +277,8 @@ int s14_moe_layer_route(s14_ctx *ctx, void *stream, const s14_router *router,
  * An EXACT block of T >= 7 runs half of its pairs on the context's own side
  * stream, joined back into `stream` (event wait) before the output is
  * written: work queued on `stream` afterwards sees y complete, and a graph
- * capture of `stream` takes the side branch in. */
+ * capture of `stream` takes the side branch in.  Under capture EXACT blocks of
+ * 5 and official blocks of 7 and 8 (8 with an MXFP4 shared page) do the same. */
 int s14_moe_block_route(s14_ctx *ctx, void *stream, uint32_t tokens, const s14_router *router,
                         const uint64_t *expert_pages_dev, const uint8_t *shared_page,
                         int shared_format, const float *x, float *y, uint16_t *ids_out,

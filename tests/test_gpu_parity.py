@@ -485,6 +485,70 @@ def test_moe_block_graph_replays(ctx, bank):
     del g
 
 
+def _kernel_nodes(launch) -> int:
+    """Kernel nodes of a HIP graph captured around launch() (never run)."""
+    import ctypes as C
+
+    with open("/proc/self/maps") as f:
+        path = next(ln.split()[-1] for ln in f if "libamdhip64" in ln)
+    hip = C.CDLL(path)
+    stream = torch.cuda.Stream()
+    graph, count = C.c_void_p(), C.c_size_t()
+    with torch.cuda.stream(stream):
+        assert hip.hipStreamBeginCapture(C.c_void_p(stream.cuda_stream), C.c_int(2)) == 0  # relaxed
+        try:
+            launch()
+        finally:
+            rc = hip.hipStreamEndCapture(C.c_void_p(stream.cuda_stream), C.byref(graph))
+    assert rc == 0 and hip.hipGraphGetNodes(graph, None, C.byref(count)) == 0
+    nodes = (C.c_void_p * count.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, C.byref(count)) == 0
+    kinds = []
+    for node in nodes:
+        kind = C.c_int()
+        assert hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0
+        kinds.append(kind.value)
+    assert hip.hipGraphDestroy(graph) == 0
+    return kinds.count(0)  # hipGraphNodeTypeKernel
+
+
+@pytest.mark.parametrize("mode,tokens,fp8,streams", [
+    (s14.EXACT, 4, False, 1), (s14.EXACT, 5, False, 2), (s14.EXACT, 6, False, 1), (s14.EXACT, 7, True, 2),
+    (s14.OFFICIAL, 5, False, 1), (s14.OFFICIAL, 7, False, 2), (s14.OFFICIAL, 7, True, 2),
+    (s14.OFFICIAL, 8, False, 2), (s14.OFFICIAL, 8, True, 1)])
+def test_moe_block_graph_streams(ctx, bank, mode, tokens, fp8, streams):
+    """The blocks that run as two halves on two streams in a captured graph
+    (where the branches cost no event latency, unlike eagerly): two launches of
+    either phase instead of one, and replays equal to the eager launch bit for
+    bit, with eager launches between them."""
+    say(f"block T={tokens} mode={mode} fp8={fp8} in a graph")
+    router = s14.Router(bank["wr_d"], bank["bias_d"])
+    shared = dev(synth.gen_fp8_page(0, 0)) if fp8 else bank["pages"][256]
+    blocks = [synth.block_tokens(seed=60 + i, tokens=tokens) for i in range(3)]
+    x_static = dev(blocks[0])
+    y_graph = torch.empty((tokens, HIDDEN), dtype=torch.float32, device="cuda")
+    y_eager = torch.empty_like(y_graph)
+
+    def launch(x, y):
+        s14.moe_block_route(ctx, tokens, router, bank["table"], shared, x, y, mode=mode,
+                            shared_format=N.S14_PAGE_FP8 if fp8 else N.S14_PAGE_MXFP4)
+
+    launch(x_static, y_graph)
+    torch.cuda.synchronize()
+    assert _kernel_nodes(lambda: launch(x_static, y_graph)) == 2 + 2 * streams
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        launch(x_static, y_graph)
+    for i, xs in enumerate(blocks):
+        x_static.copy_(dev(xs))
+        g.replay()
+        torch.cuda.synchronize()
+        got = host(y_graph)
+        launch(dev(xs), y_eager)
+        assert_bit_exact(got, host(y_eager), f"graph replay {i}")
+    del g
+
+
 def test_moe_block_on_caller_stream(ctx, bank):
     """An EXACT block launched on a caller's own stream (not torch's current
     one), with that stream's earlier work writing the block's input: the side
