@@ -101,6 +101,7 @@ def parse():
     ap.add_argument("--profile-steps", type=int, default=64)
     ap.add_argument("--cpu-seconds", type=float, default=12.0, help="bound on the CPU baseline's work per config")
     ap.add_argument("--no-cpu-baseline", action="store_true")
+    ap.add_argument("--detail", default="", help="also write the report with every timing record to this file")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="only run a plain 256 MiB device copy 10 times (the known-size kernel that "
                          "scales the FETCH_SIZE / WRITE_SIZE counters) and exit")
@@ -221,6 +222,39 @@ class Timer:
         per, host, n, cov = self._trials(graphs[1].replay, graphs[0].replay)
         del graphs
         return self._summary(per, host, n, cov, launches, launches_per_trial=launches, timing="hip graph replay")
+
+
+LINE_LIMIT = 8000  # characters of the report a reader of the output's end may count on
+
+
+def report(line: dict) -> str:
+    """The one-line JSON report: the top-level numbers as measured; in the legs
+    five significant digits, the trials as their range, and no share of the
+    HBM peak (hbm_gbps over roofline.peak).  --detail keeps all of it.  With
+    every leg's full timing record the line was 20 KB."""
+
+    def short(v):
+        if isinstance(v, float):
+            return float(f"{v:.5g}")
+        if isinstance(v, (list, tuple)):
+            return [short(e) for e in v]
+        if not isinstance(v, dict):
+            return v
+        out = {}
+        for key, e in v.items():
+            if key == "timing" and isinstance(e, dict):
+                out["ms_range"] = [short(e["ms_min"]), short(e["ms_max"])]
+                if "eager" in e:
+                    out["eager_ms"] = short(e["eager"]["ms"])
+                if not all(t["submission_covered"] for t in (e, e.get("eager", e))):
+                    out["submission_covered"] = False
+            elif key not in ("hbm_frac", "algorithmic_bytes", "n", "k", "m"):
+                out[key] = short(e)
+        return out
+
+    keep = ("config", "roofline")
+    out = {k: short(v) if isinstance(v, dict) and k not in keep else v for k, v in line.items()}
+    return json.dumps(out, separators=(",", ":"))
 
 
 def main() -> int:
@@ -423,8 +457,7 @@ def main() -> int:
             "parity": "bit-identical to the CPU oracle" if args.mode == "exact" else "order-changed f32",
             "timing": f"median of {args.trials} trials, each one replay of a HIP graph of {args.steps} steps "
                       "between two events queued behind an untimed pre-roll of the same steps (the events "
-                      "bracket the device's work; the eager figure, one host launch sequence per step, is in "
-                      "k1.timing.eager)",
+                      "bracket the device's work; the eager figure, one host launch sequence per step, is k1.eager_ms)",
             "layer_banks": NL,
             "tokens_rotated": P,
             "layer_bytes_k1": layer_bytes_k1(),
@@ -443,7 +476,10 @@ def main() -> int:
         "roofline": roofline,
         "cpu_baseline": cpu,
     }
-    print(json.dumps(line), flush=True)
+    if args.detail:
+        with open(args.detail, "w") as f:
+            json.dump(line, f, indent=1)
+    print(report(line), flush=True)
     ctx.synchronize()
     return 0
 
