@@ -1424,7 +1424,6 @@ static hipError_t launch_exact_plan(hipStream_t s, const LinearArgs &a, const Li
     case 404u: return launch_exact_mfma<4, 1, 4>(s, a);
     case 416u: return launch_exact_mfma<4, 1, 16>(s, a);
     case 804u: return launch_exact_mfma<4, 2, 4>(s, a);
-    case 808u: return launch_exact_mfma<4, 2, 8>(s, a);
     case 1604u: return launch_exact_mfma<16, 1, 4>(s, a);
     case 1608u: return launch_exact_mfma<16, 1, 8>(s, a);
     case 3204u: return launch_exact_mfma<32, 1, 4>(s, a);

@@ -113,15 +113,17 @@ struct LinExactPlan {
   uint32_t tokens, waves;
   uint64_t ns;  // estimated
 };
+struct LinExactKind {
+  uint32_t tokens, waves, alone_ns, shared_ns;
+};
+// (8 tokens on 8 wavefronts was the fastest at no size: 16 wavefronts of four
+// tokens or 4 of eight are.)
+constexpr LinExactKind kLinExactKinds[] = {{4, 4, 1760, 1110},  {4, 16, 1220, 1420}, {8, 4, 3000, 1900},
+                                           {16, 4, 3200, 2600}, {16, 8, 2650, 2850}, {32, 4, 5300, 4660}};
 inline LinExactPlan lin_exact_plan(uint32_t m, uint32_t n, uint32_t G) {
-  struct Kind {
-    uint32_t tokens, waves, alone_ns, shared_ns;
-  };
-  constexpr Kind kinds[] = {{4, 4, 1760, 1110},  {4, 16, 1220, 1420}, {8, 4, 3000, 1900},  {8, 8, 2400, 2500},
-                            {16, 4, 3200, 2600}, {16, 8, 2650, 2850}, {32, 4, 5300, 4660}};
   const uint64_t tiles = (uint64_t(n) + 63u) / 64u;
   LinExactPlan best{0, 0, ~uint64_t(0)};
-  for (const Kind &k : kinds) {
+  for (const LinExactKind &k : kLinExactKinds) {
     const uint64_t wgs = tiles * ((uint64_t(m) + k.tokens - 1u) / k.tokens);
     const uint64_t t = (wgs + 255u) / 256u * ((G + k.waves - 1u) / k.waves) * (k.waves / 4u) *
                        (wgs <= 256u ? k.alone_ns : k.shared_ns);

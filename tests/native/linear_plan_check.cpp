@@ -33,3 +33,17 @@ extern "C" uint32_t lin_exact(uint32_t m, uint32_t n, uint32_t groups, uint32_t 
   *waves = p.waves;
   return s14::lin_exact_first(m, n, groups);
 }
+
+// Bit i: kind i of the EXACT f32-MFMA plan is the fastest at some size.
+extern "C" uint32_t lin_exact_kinds(uint32_t *count) {
+  *count = uint32_t(sizeof(s14::kLinExactKinds) / sizeof(s14::kLinExactKinds[0]));
+  uint32_t seen = 0;
+  for (uint32_t tiles = 1; tiles <= 600; ++tiles)
+    for (uint32_t groups = 1; groups <= 1024; groups += groups < 64 ? 1 : 64)
+      for (uint32_t m = 2; m <= 300; ++m) {
+        const s14::LinExactPlan p = s14::lin_exact_plan(m, 64 * tiles, groups);
+        for (uint32_t i = 0; i < *count; ++i)
+          if (s14::kLinExactKinds[i].tokens == p.tokens && s14::kLinExactKinds[i].waves == p.waves) seen |= 1u << i;
+      }
+  return seen;
+}

@@ -114,7 +114,7 @@ def test_prompt_tile_and_exact_mfma_plans(plan_lib, n, k):
     of whole 32-token blocks)."""
     groups = k // 128
     a, b = C.c_uint32(), C.c_uint32()
-    kinds = {(4, 4), (4, 16), (8, 4), (8, 8), (16, 4), (16, 8), (32, 4)}
+    kinds = {(4, 4), (4, 16), (8, 4), (16, 4), (16, 8), (32, 4)}
     for m in [*range(1, 400), 511, 512, 513, 1023, 1024, 5000]:
         plan_lib.lin_gemm(C.c_uint32(m), C.c_uint32(n), C.c_uint32(groups), C.byref(a), C.byref(b))
         tokens, splits = a.value, b.value
@@ -129,3 +129,10 @@ def test_prompt_tile_and_exact_mfma_plans(plan_lib, n, k):
         for part in {first, m - first} - {0}:
             plan_lib.lin_exact(C.c_uint32(part), C.c_uint32(n), C.c_uint32(groups), C.byref(a), C.byref(b))
             assert (a.value, b.value) in kinds
+
+
+def test_every_exact_mfma_kind_is_chosen(plan_lib):
+    """No kernel of the EXACT f32-MFMA plan is built for nothing."""
+    count = C.c_uint32()
+    seen = plan_lib.lin_exact_kinds(C.byref(count))
+    assert seen == (1 << count.value) - 1, bin(seen)
