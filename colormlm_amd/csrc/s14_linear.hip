@@ -805,7 +805,7 @@ __global__ __launch_bounds__(64 * kLgWaves) void k_linear_gemm(LinearArgs a, flo
 // and accumulates; the wavefront sum (DPP) gives the row.  (Splitting k
 // across wavefronts instead, with the split partials met as k_linear_fast
 // meets them, was slower at wo_a and wo_b: 13.3 and 14.9 us.)
-constexpr uint32_t kGvChunk = 1024, kGvLoads = 8, kGvWaves = 4;
+constexpr uint32_t kGvChunk = kLinGvChunk, kGvLoads = 8, kGvWaves = 4;
 template <int MT, int R, bool kXsF32, bool kWsF32>
 __global__ __launch_bounds__(64 * kGvWaves) void k_linear_gemv(LinearArgs a) {
   constexpr uint32_t kB = kGvLoads / uint32_t(R);  // chunks per batch
@@ -1431,92 +1431,83 @@ static hipError_t launch_exact_plan(hipStream_t s, const LinearArgs &a, const Li
   }
 }
 
-hipError_t launch_fp8_linear(hipStream_t s, const LinearArgs &a, int mode, const LinearWorkspace &ws) {
-  // the GEMV where it measured faster than the MFMA tiles (graph replays,
-  // us: wq_b m = 1 8.5 against 10.4, m = 2 10.9 against 10.7; wo_a m = 2 11.2
-  // against 12.6, m = 3 14.7 against 13.1; wkv m = 4 4.9 against 7.9)
-  const bool gemv = a.m == 1u || (a.m == 2u && a.n <= 8192u) || (a.m <= 4u && a.n <= 1024u);
-  if (mode == S14_MODE_FAST && gemv && a.k % kGvChunk == 0u && uint64_t(a.n) * a.k <= 0xFFFFFFFFull) {
-    if (a.m == 1)
-      launch_gemv_mt<1>(s, a);
-    else if (a.m == 2)
-      launch_gemv_mt<2>(s, a);
-    else
-      launch_gemv_mt<4>(s, a);
-    return hipGetLastError();
-  }
-  const bool fast = mode == S14_MODE_FAST && a.k % (4u * kLinGroup) == 0u;
-  // the prompt tiles from where they measured faster than k_linear_fast
-  // (us: wq_b m = 8 11.7 against 12.0, m = 12 17.9 against 11.9; wo_b m = 12 24.3
-  // against 13.8; wkv m = 64 14.6 against 17.8, m = 333 27.6 against 17.9)
-  if (fast && a.m > 8u && uint64_t(a.m) * a.n * a.k >= 300000000ull && uint64_t(a.n + kLgRows - 1) * a.k <= 0xFFFFFFFFull) {
-    const LinGemmPlan p = lin_gemm_plan(a.m, a.n, a.groups);
-    float *part = p.splits > 1u ? ws.part : nullptr;
-    if (p.tokens == 32u)
-      launch_gemm_tt<2>(s, a, part, p.splits);
-    else
-      launch_gemm_tt<4>(s, a, part, p.splits);
-    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    if (part) launch_sum(s, a, part, p.splits);
-    return hipGetLastError();
-  }
-  const LinFastPlan plan = fast ? lin_fast_plan(a.m, a.n, a.groups) : LinFastPlan{0, 0};
-  if (plan.cw) {
-    // one launch per plan.blocks token blocks, each within the workspace's
-    // partials and counters (a smaller last launch fits whatever fits more)
-    const uint32_t tiles = (a.n + kLinTile - 1) / kLinTile, per = plan.blocks * kLinTile;
-    const uint32_t xs_stride = a.x_scale_f32 ? 4u : 1u;
-    for (uint32_t m0 = 0; m0 < a.m; m0 += per) {
-      LinearArgs c = a;
-      c.m = std::min(per, a.m - m0);
-      c.x = a.x + size_t(m0) * a.k;
-      c.x_scale = static_cast<const uint8_t *>(a.x_scale) + size_t(m0) * a.groups * xs_stride;
-      c.y = a.y + size_t(m0) * a.n;
-      const uint32_t ncb = (c.m + kLinTile - 1) / kLinTile, ntok = std::min(c.m, kLinTile);
-      const uint32_t cw = lin_fast_chunks(a.groups, tiles, ncb, ntok);
-      const uint32_t splits = cw ? a.groups / cw : 0u;
-      if (!cw || lin_part_bytes(tiles, ncb, splits) > kLinPartBytes ||
-          (splits > 1u && uint64_t(tiles) * ncb > kLinMaxCounters))
-        return hipErrorInvalidValue;  // unreachable: the plan fits every launch
-      launch_fast_ring<kLinRing>(s, c, ws, cw, splits, dim3(tiles, splits, ncb), lin_stage_bytes(ntok, cw));
-      if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    }
-    return hipSuccess;
-  }
-  const bool vec = a.k % 16u == 0u &&
-                   ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.w)) & 15u) == 0u;
-  if (a.m == 1u && vec && uint64_t(a.n) * a.k <= 0xFFFFFFFFull &&
-      (a.k == 1024u || a.k == 2048u || a.k == 4096u || a.k == 8192u)) {
-    switch (a.k) {
-      case 1024u: launch_gemv_exact<8>(s, a); break;
-      case 2048u: launch_gemv_exact<4>(s, a); break;
-      case 4096u: launch_gemv_exact<2>(s, a); break;
-      default: launch_gemv_exact<1>(s, a); break;
-    }
-    return hipGetLastError();
-  }
-  // the f32 MFMA: UE8M0 scales, whole groups.  Two to four tokens over a k
-  // past 4,096 stay on the tiles below (wo_b m = 4: 21.5 us against 24.1:
-  // 64-row workgroups leave most CUs idle there)
-  if (vec && a.k % kLinGroup == 0u && !a.x_scale_f32 && !a.w_scale_f32 && (a.m > 4u || a.k <= 4096u) &&
-      uint64_t(a.n + kXmRows - 1) * a.k <= 0xFFFFFFFFull &&
-      !(size_t(a.groups) * a.n * sizeof(float) <= kLinPartBytes && lin_exact_tiles(a.m, a.n, a.groups))) {
-    const uint32_t first = lin_exact_first(a.m, a.n, a.groups);
+// EXACT on the f32 MFMA, in one launch or two (lin_exact_first).
+static hipError_t launch_exact_mfma_plans(hipStream_t s, const LinearArgs &a) {
+  const uint32_t first = lin_exact_first(a.m, a.n, a.groups);
+  LinearArgs c = a;
+  c.m = first;
+  const hipError_t e = launch_exact_plan(s, c, lin_exact_plan(c.m, c.n, c.groups));
+  if (e != hipSuccess || first == a.m) return e;
+  c.m = a.m - first;
+  c.x = a.x + size_t(first) * a.k;
+  c.x_scale = static_cast<const uint8_t *>(a.x_scale) + size_t(first) * a.groups;
+  c.y = a.y + size_t(first) * a.n;
+  return launch_exact_plan(s, c, lin_exact_plan(c.m, c.n, c.groups));
+}
+
+static hipError_t launch_gemm(hipStream_t s, const LinearArgs &a, const LinearWorkspace &ws) {
+  const LinGemmPlan p = lin_gemm_plan(a.m, a.n, a.groups);
+  float *part = p.splits > 1u ? ws.part : nullptr;
+  if (p.tokens == 32u)
+    launch_gemm_tt<2>(s, a, part, p.splits);
+  else
+    launch_gemm_tt<4>(s, a, part, p.splits);
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  if (part) launch_sum(s, a, part, p.splits);
+  return hipGetLastError();
+}
+
+// k_linear_fast, one launch per plan.blocks token blocks, each within the
+// workspace's partials and counters (a smaller last launch fits whatever fits
+// more)
+static hipError_t launch_fast(hipStream_t s, const LinearArgs &a, const LinearWorkspace &ws) {
+  const LinFastPlan plan = lin_fast_plan(a.m, a.n, a.groups);
+  const uint32_t tiles = (a.n + kLinTile - 1) / kLinTile, per = plan.blocks * kLinTile;
+  const uint32_t xs_stride = a.x_scale_f32 ? 4u : 1u;
+  for (uint32_t m0 = 0; m0 < a.m; m0 += per) {
     LinearArgs c = a;
-    c.m = first;
-    const hipError_t e = launch_exact_plan(s, c, lin_exact_plan(c.m, c.n, c.groups));
-    if (e != hipSuccess || first == a.m) return e;
-    c.m = a.m - first;
-    c.x = a.x + size_t(first) * a.k;
-    c.x_scale = static_cast<const uint8_t *>(a.x_scale) + size_t(first) * a.groups;
-    c.y = a.y + size_t(first) * a.n;
-    return launch_exact_plan(s, c, lin_exact_plan(c.m, c.n, c.groups));
+    c.m = std::min(per, a.m - m0);
+    c.x = a.x + size_t(m0) * a.k;
+    c.x_scale = static_cast<const uint8_t *>(a.x_scale) + size_t(m0) * a.groups * xs_stride;
+    c.y = a.y + size_t(m0) * a.n;
+    const uint32_t ncb = (c.m + kLinTile - 1) / kLinTile, ntok = std::min(c.m, kLinTile);
+    const uint32_t cw = lin_fast_chunks(a.groups, tiles, ncb, ntok);
+    const uint32_t splits = cw ? a.groups / cw : 0u;
+    if (!cw || lin_part_bytes(tiles, ncb, splits) > kLinPartBytes ||
+        (splits > 1u && uint64_t(tiles) * ncb > kLinMaxCounters))
+      return hipErrorInvalidValue;  // unreachable: the plan fits every launch
+    launch_fast_ring<kLinRing>(s, c, ws, cw, splits, dim3(tiles, splits, ncb), lin_stage_bytes(ntok, cw));
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   }
-  // tiled: whole groups, one token's partials within the workspace, and the
-  // last tile's row offsets within 32 bits (rows past n read zeros)
-  if (vec && a.k % kLinGroup == 0u && size_t(a.groups) * a.n * sizeof(float) <= kLinPartBytes &&
-      uint64_t(a.n + kLTRows - 1) * a.k <= 0xFFFFFFFFull)
-    return launch_exact_tiled(s, a, ws);
+  return hipSuccess;
+}
+
+hipError_t launch_fp8_linear(hipStream_t s, const LinearArgs &a, int mode, const LinearWorkspace &ws) {
+  const bool aligned = ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.w)) & 15u) == 0u;
+  switch (lin_route(mode == S14_MODE_FAST, a.m, a.n, a.k, a.x_scale_f32 || a.w_scale_f32, aligned)) {
+    case LinRoute::kGemv:
+      if (a.m == 1)
+        launch_gemv_mt<1>(s, a);
+      else if (a.m == 2)
+        launch_gemv_mt<2>(s, a);
+      else
+        launch_gemv_mt<4>(s, a);
+      return hipGetLastError();
+    case LinRoute::kGemm: return launch_gemm(s, a, ws);
+    case LinRoute::kFast: return launch_fast(s, a, ws);
+    case LinRoute::kGemvExact:
+      switch (a.k) {
+        case 1024u: launch_gemv_exact<8>(s, a); break;
+        case 2048u: launch_gemv_exact<4>(s, a); break;
+        case 4096u: launch_gemv_exact<2>(s, a); break;
+        default: launch_gemv_exact<1>(s, a); break;
+      }
+      return hipGetLastError();
+    case LinRoute::kExactMfma: return launch_exact_mfma_plans(s, a);
+    case LinRoute::kTile: return launch_exact_tiled(s, a, ws);
+    case LinRoute::kExact: break;
+  }
+  const bool vec = a.k % 16u == 0u && aligned;
   if (a.m == 1) return launch_exact_mt<1>(s, a, vec);
   if (a.m == 2) return launch_exact_mt<2>(s, a, vec);
   if (a.m <= 4) return launch_exact_mt<4>(s, a, vec);

@@ -1,8 +1,11 @@
-// Launch planning of the FAST fp8_linear (k_linear_fast): how many 128-k
-// chunks each wavefront streams (its K split is groups / cw) and how many
-// 32-token blocks one launch takes, so that the split-K partials and the
-// arrival counters always fit the context's linear workspace.  Plain C++ (no
-// HIP types): the library and a host-only test include it.
+// Launch planning of fp8_linear: which kernel takes a call (lin_route) and its
+// sizes.  FAST: how many 128-k chunks each wavefront of k_linear_fast streams
+// (its K split is groups / cw) and how many 32-token blocks one launch takes,
+// so that the split-K partials and the arrival counters always fit the
+// context's linear workspace; the K splits of k_linear_gemm.  EXACT: the tile
+// of k_linear_exact_mfma, and the tokens of a first launch where two are
+// faster.  Plain C++ (no HIP types): the library and a host-only test include
+// it.
 #pragma once
 
 #include <cstddef>
@@ -88,8 +91,8 @@ inline LinGemmPlan lin_gemm_plan(uint32_t m, uint32_t n, uint32_t G) {
   uint64_t least = ~uint64_t(0);
   for (uint32_t s : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u, 24u, 32u}) {
     const uint64_t part = uint64_t(m) * n * s * sizeof(float), per = (G + s - 1u) / s;
-    // at least four groups a split (as k_linear_fast has: more partial sums
-    // round more often), and none without any
+    // four groups a split or more (as k_linear_fast has: more partial sums
+    // round more often); the last one takes what is left, at least one
     if (s > 1u && (part > kLinPartBytes || per < 4u || uint64_t(s - 1u) * per >= G)) continue;
     const uint64_t wgs = tiles * s;
     const uint64_t t = (wgs <= 256u ? alone : (wgs + 511u) / 512u * shared) * per +
@@ -163,6 +166,44 @@ inline bool lin_exact_tiles(uint32_t m, uint32_t n, uint32_t G) {
   const uint64_t waves = (uint64_t(n) + 63u) / 64u * G * ((uint64_t(m) + 7u) / 8u);
   const uint64_t first = m <= 2u ? 5600u : m <= 4u ? 6800u : 9500u, more = m <= 2u ? 2200u : m <= 4u ? 3000u : 5200u;
   return first + (waves + 1023u) / 1024u * more - more < lin_exact_plan(m, n, G).ns + 2000u;
+}
+
+// The kernel that takes a call.  `aligned`: x and w start at 16-byte addresses.
+constexpr uint32_t kLinGvChunk = 1024;  // k per chunk of k_linear_gemv
+enum class LinRoute : uint32_t {
+  kGemv,       // FAST, few tokens: k_linear_gemv
+  kGemm,       // FAST prompts: k_linear_gemm
+  kFast,       // FAST otherwise: k_linear_fast
+  kGemvExact,  // one token: k_linear_gemv_exact
+  kExactMfma,  // UE8M0 scales on both sides: k_linear_exact_mfma
+  kTile,       // k_linear_tile + k_linear_sum
+  kExact,      // any other: k_linear_exact
+};
+inline LinRoute lin_route(bool fast, uint32_t m, uint32_t n, uint32_t k, bool f32_scales, bool aligned) {
+  constexpr uint64_t kMax32 = 0xFFFFFFFFull;  // row offsets, of the last tile's rows past n too
+  const uint32_t G = (k + kLinGroup - 1u) / kLinGroup;
+  // the GEMV where it measured faster than the MFMA tiles (graph replays,
+  // us: wq_b m = 1 8.5 against 10.4, m = 2 10.9 against 10.7; wo_a m = 2 11.2
+  // against 12.6, m = 3 14.7 against 13.1; wkv m = 4 4.9 against 7.9)
+  const bool gemv = m == 1u || (m == 2u && n <= 8192u) || (m <= 4u && n <= 1024u);
+  if (fast && gemv && k % kLinGvChunk == 0u && uint64_t(n) * k <= kMax32) return LinRoute::kGemv;
+  if (fast && k % (4u * kLinGroup) == 0u) {
+    // the prompt tiles from where they measured faster than k_linear_fast
+    // (us: wq_b m = 8 11.7 against 12.0, m = 12 17.9 against 11.9; wo_b m = 12 24.3
+    // against 13.8; wkv m = 64 14.6 against 17.8, m = 333 27.6 against 17.9)
+    if (m > 8u && uint64_t(m) * n * k >= 300000000ull && (uint64_t(n) + 127u) * k <= kMax32) return LinRoute::kGemm;
+    if (lin_fast_plan(m, n, G).cw) return LinRoute::kFast;
+  }
+  const bool vec = k % 16u == 0u && aligned;
+  if (m == 1u && vec && uint64_t(n) * k <= kMax32 && (k == 1024u || k == 2048u || k == 4096u || k == 8192u))
+    return LinRoute::kGemvExact;
+  if (!vec || k % kLinGroup != 0u || (uint64_t(n) + 63u) * k > kMax32) return LinRoute::kExact;
+  const bool tile = size_t(G) * n * sizeof(float) <= kLinPartBytes;  // one token's partials fit the workspace
+  // the f32 MFMA: UE8M0 scales, whole groups.  Two to four tokens over a k
+  // past 4,096 stay on the tiles (wo_b m = 4: 21.5 us against 24.1: 64-row
+  // workgroups leave most CUs idle there)
+  if (!f32_scales && (m > 4u || k <= 4096u) && !(tile && lin_exact_tiles(m, n, G))) return LinRoute::kExactMfma;
+  return tile ? LinRoute::kTile : LinRoute::kExact;
 }
 
 }  // namespace s14

@@ -25,6 +25,19 @@ pytestmark = pytest.mark.gpu
 SHAPES = {"wq_b": (32768, 1024), "wkv": (512, 4096), "wo_a": (8192, 4096), "wo_b": (4096, 8192)}
 
 
+# The tests below that name a kernel, with the shapes that reach it: test_linear_plan.py
+# holds each to that kernel by the library's own rule.  (m, n, k[, f32 scales])
+EXACT_MFMA = [(2, 300, 384), (3, 64, 128), (5, 4160, 1152), (13, 1000, 640), (17, 8192, 256), (31, 2000, 1536),
+              (33, 16450, 512), (65, 700, 2176), (97, 8200, 384), (160, 12288, 256), (52, 4160, 640), (132, 1000, 640),
+              (12, 8192, 2048), (65, 8192, 2048), (9, 1967, 3200), (23, 7239, 1664), (65, 9982, 1152),
+              (52, 4131, 640), (33, 16450, 640), (40, 32768, 1024)]
+EXACT_TILE_CHUNKS = [(40, 32768, 1024, True), (7, 129, 4096, False)]
+FAST_PROMPT = [(9, 33000, 1024, False), (31, 8192, 1536, True), (33, 4099, 4096, False), (64, 1030, 8192, True),
+               (65, 8200, 1024, False), (200, 512, 4096, False), (333, 700, 2560, True), (129, 32768, 1024, False),
+               (512, 32768, 1024, False)]
+FAST_LAUNCHES = [(1100, 2, 131072, False), (1060, 2, 131072, True)]
+
+
 def say(msg: str) -> None:
     print(f"[gpu-test] {msg}", file=sys.stderr, flush=True)
 
@@ -67,10 +80,11 @@ def decoded(oracle, c, scales, row_group):
     return lut[c] * s
 
 
-def check_fast(oracle, got, want, x, xs, w, ws, what):
+def check_fast(oracle, got, want, x, xs, w, ws, what, l1=None):
     """|fast - oracle| <= 2e-6 * sum_k |x_k w_k| of the row (f32 summation
     error; measured <= 3.2e-7)."""
-    l1 = np.abs(decoded(oracle, x, xs, 1)) @ np.abs(decoded(oracle, w, ws, 128)).T
+    if l1 is None:
+        l1 = np.abs(decoded(oracle, x, xs, 1)) @ np.abs(decoded(oracle, w, ws, 128)).T
     err = np.abs(got.astype(np.float64) - want)
     ratio = float(np.max(err / np.maximum(l1, 1e-30)))
     say(f"  {what}: fast max |err| / row L1 = {ratio:.3g}")
@@ -262,18 +276,15 @@ def test_fp8_linear_exact_one_token_extreme_scales(ctx, oracle, k):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.count_nonzero(got != want)
 
 
-@pytest.mark.parametrize("m,n,k", [(2, 300, 384), (3, 64, 128), (5, 4160, 1152), (7, 129, 4096), (13, 1000, 640),
-                                   (17, 8192, 256), (31, 2000, 1536), (33, 16450, 512), (65, 700, 2176),
-                                   (97, 8200, 384), (160, 12288, 256),
-                                   (52, 4160, 640), (132, 1000, 640), (12, 8192, 2048),
-                                   (65, 8192, 2048)])
+@pytest.mark.parametrize("m,n,k", EXACT_MFMA)
 def test_fp8_linear_exact_mfma_plans(ctx, oracle, m, n, k):
     """The f32-MFMA EXACT kernel with every plan (4, 8, 16 and 32 tokens per
-    workgroup; 4, 8 and 16 wavefronts; m = 65 in two launches): rows cut inside a 64-row tile,
-    tokens cut inside a block, fewer groups than wavefronts and a ragged last
-    round of groups; then UE8M0 codes that leave the MFMA's window (0..12, so
-    that products fall to subnormals or zero), a bias and bf16 outputs; bit
-    for bit."""
+    workgroup; 4, 8 and 16 wavefronts; m = 65 at k = 2,048 in two launches),
+    each also over several rounds of groups with a ragged last one: rows cut
+    inside a 64-row tile, tokens cut inside a block, fewer groups than
+    wavefronts; then UE8M0 codes that leave the MFMA's window (0..12, so that
+    products fall to subnormals or zero), a bias and bf16 outputs; bit for
+    bit."""
     say(f"fp8_linear exact mfma m={m} n={n} k={k}")
     rng = np.random.default_rng(m * n + k)
     w, x = codes(rng, (n, k)), codes(rng, (m, k))
@@ -293,24 +304,54 @@ def test_fp8_linear_exact_mfma_plans(ctx, oracle, m, n, k):
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (extreme, np.count_nonzero(got != want))
 
 
-def test_fp8_linear_exact_token_chunks(ctx, oracle):
-    """EXACT keeps every group partial of a launch in the context's 32 MiB
-    workspace: at wq_b's shape (8 groups x 32768 rows x 4 bytes per token)
-    40 tokens take two launches of the tiled kernel, 32 tokens then 8."""
-    say("fp8_linear exact token chunks: wq_b m=40")
-    n, k, m = 32768, 1024, 40
+@pytest.mark.parametrize("f32", [False, True])
+def test_fp8_linear_exact_upper_scales(ctx, oracle, f32):
+    """Scale codes at the upper ends of the windows, UE8M0 on both sides: the
+    codes' sum on both sides of 356 (f32 MFMA, 5 tokens) and of 364 (one token),
+    a code on both sides of 246; e4m3 codes below 2^-1 keep every product and sum
+    finite.  The same values as f32 scales on the tiles.  Bit for bit."""
+    say(f"fp8_linear exact, upper scale codes, f32={f32}")
+    n, k = 200, 1024
+    rng = np.random.default_rng(4)
+    w, x = rng.integers(0, 0x30, (n, k), dtype=np.uint8), rng.integers(0, 0x30, (5, k), dtype=np.uint8)
+    w, x = w | rng.choice(np.array([0, 0x80], np.uint8), w.shape), x | rng.choice(np.array([0, 0x80], np.uint8), x.shape)
+    for m, top in ((5, 356), (1, 364)):
+        for step in range(-2, 3):
+            for cw in (top - 246 - 1, top - 246, 178, 246, 247):
+                ws = np.full((2, k // 128), 120, np.uint8)
+                xs = np.full((m, k // 128), 120, np.uint8)
+                g = int(rng.integers(k // 128))
+                ws[:, g], xs[:, g] = cw, top + step - cw
+                xs[0, g] -= step > 0  # one token inside beside others outside
+                if f32:
+                    ws, xs = (np.exp2(a.astype(np.float32) - 127) for a in (ws, xs))
+                want = oracle.fp8_linear(x[:m], xs, w, ws)
+                assert np.isfinite(want).all()
+                y = torch.full((m, n), np.nan, dtype=torch.float32, device="cuda")
+                s14.fp8_linear(ctx, dev(x[:m]), dev(xs), dev(w), dev(ws), y, mode=s14.EXACT)
+                assert np.array_equal(host(y).view(np.uint32), want.view(np.uint32)), (m, step, cw)
+
+
+@pytest.mark.parametrize("m,n,k,f32", EXACT_TILE_CHUNKS)
+def test_fp8_linear_exact_token_chunks(ctx, oracle, m, n, k, f32):
+    """The tiled EXACT kernel keeps every group partial of a launch in the
+    context's 32 MiB workspace: at wq_b's shape with f32 scales (8 groups x
+    32768 rows x 4 bytes per token) 40 tokens take two launches, 32 tokens then
+    8.  And UE8M0 scales where few rows and tokens bring the call to the tiles."""
+    say(f"fp8_linear exact tiles: m={m} n={n} k={k} f32={f32}")
     w, ws = weight(n, k, seed=11)
     rng = np.random.default_rng(12)
     x, xs = codes(rng, (m, k)), rng.integers(120, 128, (m, k // 128), dtype=np.uint8)
+    if f32:
+        ws = rng.uniform(1e-3, 4e-3, ws.shape).astype(np.float32)
+        xs = rng.uniform(1e-2, 3e-2, xs.shape).astype(np.float32)
     want = oracle.fp8_linear(x, xs, w, ws)
     y = torch.empty((m, n), dtype=torch.float32, device="cuda")
     s14.fp8_linear(ctx, dev(x), dev(xs), dev(w), dev(ws), y, mode=s14.EXACT)
     assert np.array_equal(host(y).view(np.uint32), want.view(np.uint32))
 
 
-@pytest.mark.parametrize("m,n,k,f32", [(9, 33000, 1024, False), (31, 8192, 1536, True), (33, 4099, 4096, False),
-                                       (64, 1030, 8192, True), (65, 8200, 1024, False), (200, 512, 4096, False),
-                                       (333, 700, 2560, True)])
+@pytest.mark.parametrize("m,n,k,f32", FAST_PROMPT)
 def test_fp8_linear_fast_prompt_tiles(ctx, oracle, m, n, k, f32):
     """The prompt-tile FAST kernel: 32- and 64-token workgroups, rows cut by n
     inside a wavefront's and a workgroup's rows (and n not a multiple of 4:
@@ -335,17 +376,23 @@ def test_fp8_linear_fast_prompt_tiles(ctx, oracle, m, n, k, f32):
     assert np.array_equal(host(y), torch.from_numpy(got).bfloat16().float().numpy())
 
 
-@pytest.mark.parametrize("m", [129, 512])
-def test_fp8_linear_fast_token_blocks_in_several_launches(ctx, oracle, m):
-    """wq_b's FAST split-K partials take 8 MiB per 32-token block, so the
-    32 MiB workspace holds 4 blocks: 129 tokens run as launches of 96 and 33
-    tokens, 512 as four of 128.  Every token's row matches the oracle."""
-    n, k = SHAPES["wq_b"]
-    say(f"fp8_linear fast wq_b m={m} (several launches)")
-    w, ws = weight(n, k, seed=21)
+@pytest.mark.parametrize("m,n,k,f32", FAST_LAUNCHES)
+def test_fp8_linear_fast_token_blocks_in_several_launches(ctx, oracle, m, n, k, f32):
+    """k_linear_fast over a long k: 256 K splits a token block, so the 32 MiB
+    workspace holds the partials of 32 blocks and more tokens take two launches
+    (18 blocks of 35 and 17 of 34 each): x, scale and y offsets and the counters
+    between them.  Every token's row matches the oracle."""
+    say(f"fp8_linear fast m={m} n={n} k={k} f32={f32} (several launches)")
     rng = np.random.default_rng(m)
-    x, xs = codes(rng, (m, k)), rng.integers(120, 128, (m, k // 128), dtype=np.uint8)
+    w, x = codes(rng, (n, k)), codes(rng, (m, k))
+    if f32:
+        ws = rng.uniform(1e-3, 4e-3, (1, k // 128)).astype(np.float32)
+        xs = rng.uniform(1e-2, 3e-2, (m, k // 128)).astype(np.float32)
+    else:
+        ws = rng.integers(114, 122, (1, k // 128), dtype=np.uint8)
+        xs = rng.integers(120, 128, (m, k // 128), dtype=np.uint8)
     want = oracle.fp8_linear(x, xs, w, ws)
+    l1 = oracle.fp8_linear(x & 0x7F, xs, w & 0x7F, ws)  # the sum of |products|, to f32 rounding
     y = torch.full((m, n), np.nan, dtype=torch.float32, device="cuda")
     s14.fp8_linear(ctx, dev(x), dev(xs), dev(w), dev(ws), y, mode=s14.FAST)
-    check_fast(oracle, host(y), want, x, xs, w, ws, f"wq_b m={m}")
+    check_fast(oracle, host(y), want, x, xs, w, ws, f"m={m} n={n} k={k}", l1=l1)

@@ -1374,6 +1374,51 @@ def test_fp8_shared_edge_scale_codes(ctx, oracle, bank, mode, topk):
             assert_bit_exact(got[t], want, f"block token {t}")
 
 
+@pytest.mark.parametrize("mode", [s14.EXACT, s14.OFFICIAL])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_shared_page_upper_scale_codes(ctx, oracle, bank, mode, fp8):
+    """Scale codes on both sides of the upper ends of the decode windows: the
+    fused form of official blocks (376 - emax, FP8 tiles 370 - emax) and the FP8
+    tiles' 246.  Each code stands in row tiles of its own, so that a wavefront
+    whose largest code is the last inside takes the fast path; the weights under
+    it are few and small, which keeps every output finite (w1 and w3 rows
+    saturate the SwiGLU's clamp, w2 rows reach 2^127).  A block of 3 and its
+    first token alone."""
+    say(f"upper scale codes, fp8={fp8} mode={mode}")
+    o = synth.page_offsets("fp8" if fp8 else "mxfp4")
+    rng = np.random.default_rng(3)
+    sh = synth.gen_fp8_page(0, 0).copy() if fp8 else page_host(bank, 256).copy()
+    for wname, sname, n, k, codes in (("w1", "s1", INTER, HIDDEN, range(238, 250)),
+                                      ("w3", "s3", INTER, HIDDEN, range(237, 249)),
+                                      ("w2", "s2", HIDDEN, INTER, range(232, 249))):
+        for i, c in enumerate(codes):
+            if fp8:  # tile (i, i): 128 x 128 codes of +-2^-9 and +-2^-8
+                tile = rng.choice(np.array([0x01, 0x81, 0x02, 0x82], np.uint8), (128, 128))
+                j = i % (k // 128)
+                sh[o[wname]:o[sname]].reshape(n, k)[128 * i:128 * i + 128, 128 * j:128 * j + 128] = tile
+                sh[o[sname] + i * (k // 128) + j] = c
+            else:  # one weight of +-0.5 in group 3 i of a row
+                row, g = 64 * i + 5, 3 * i + 1
+                group = sh[o[wname] + (row * k + 32 * g) // 2:][:16]
+                group[:] = 0
+                group[int(rng.integers(16))] = rng.choice(np.array([0x01, 0x10, 0x09, 0x90], np.uint8))
+                sh[o[sname] + row * (k // 32) + g] = c
+    fmt = N.S14_PAGE_FP8 if fp8 else N.S14_PAGE_MXFP4
+    layer = oracle.moe_layer_official if mode == s14.OFFICIAL else oracle.moe_layer
+    xs = synth.block_tokens(seed=17, tokens=3)
+    want = []
+    for t in range(3):
+        _, i_o, w_o = oracle.route(bank["wr"], bank["bias"], xs[t])
+        want.append(layer(xs[t], [page_host(bank, int(e)) for e in i_o], w_o, sh, shared_fmt="fp8" if fp8 else "mxfp4"))
+        assert np.isfinite(want[t]).all() and np.abs(want[t]).max() > 1e36
+    router, y = s14.Router(bank["wr_d"], bank["bias_d"]), torch.empty((3, HIDDEN), dtype=torch.float32, device="cuda")
+    s14.moe_block_route(ctx, 3, router, bank["table"], dev(sh), dev(xs), y, shared_format=fmt, mode=mode)
+    for t in range(3):
+        assert_bit_exact(host(y)[t], want[t], f"block token {t}")
+    s14.moe_layer_route(ctx, router, bank["table"], dev(sh), dev(xs[0]), y[0], shared_format=fmt, mode=mode)
+    assert_bit_exact(host(y)[0], want[0], "layer")
+
+
 def test_official_chain_weight_before_w2(ctx, oracle, bank):
     """The expert chain in official mode: one routed expert, its weight on h
     before w2, no shared expert."""

@@ -1,11 +1,12 @@
-"""The FAST fp8_linear's launch plan (csrc/s14_linear_plan.h), compiled for
-the host: every launch it makes keeps its split-K partials within the
-context's 32 MiB workspace and its (row tile, token block) arrival counters
-within the 65,536 the workspace holds, its staged activations within the
-wavefront's LDS budget, and its K split whole (chunk widths are multiples
-of 4 dividing the group count).  Checked for m = 1..1024 tokens at the
-adjacent projections' shapes (l42_reference.py:89-102) and at shapes that
-force the token blocks into several launches or FAST off altogether."""
+"""fp8_linear's launch plans (csrc/s14_linear_plan.h), compiled for the host.
+k_linear_fast: every launch keeps its split-K partials within the context's
+32 MiB workspace and its (row tile, token block) arrival counters within the
+65,536 the workspace holds, its staged activations within the wavefront's LDS
+budget, and its K split whole (chunk widths are multiples of 4 dividing the
+group count), for m = 1..1024 tokens at the adjacent projections' shapes
+(l42_reference.py:89-102) and at shapes that force the token blocks into
+several launches or FAST off altogether.  The prompt tiles' and the EXACT
+f32-MFMA kernel's plans, and the kernel that each shape of the GPU tests takes."""
 
 from __future__ import annotations
 
@@ -41,8 +42,8 @@ def plan_lib(tmp_path_factory):
 
 
 def launches(lib, m, n, k):
-    """The launches launch_fp8_linear makes: [(tokens, chunk width, splits)]
-    or None when FAST hands the shape to EXACT."""
+    """The launches of k_linear_fast: [(tokens, chunk width, splits)], or None
+    for a shape that it cannot take."""
     groups = -(-k // 128)
     cw, blocks = C.c_uint32(), C.c_uint32()
     lib.lin_plan(m, n, groups, C.byref(cw), C.byref(blocks))
@@ -81,13 +82,13 @@ def test_fast_plan_fits_the_workspace_for_every_token_count(plan_lib, name):
     n, k = SHAPES[name]
     for m in range(1, 1025):
         plan = check(plan_lib, m, n, k)
-        # the projections always run FAST (a shape FAST cannot plan goes to EXACT)
+        # the projections always plan (a shape that FAST cannot plan goes to EXACT)
         assert plan is not None, (name, m)
 
 
 def test_fast_plan_splits_token_blocks_where_partials_would_overflow(plan_lib):
-    # wq_b: 1,024 row tiles x 2 splits x 4 KiB = 8 MiB of partials per token
-    # block, so at most 4 blocks (128 tokens) per launch
+    # 1,024 row tiles x 2 splits x 4 KiB = 8 MiB of partials per token block, so
+    # at most 4 blocks (128 tokens) per launch
     assert launches(plan_lib, 128, 32768, 1024) == [(128, 4, 2)]
     assert launches(plan_lib, 129, 32768, 1024) == [(96, 4, 2), (33, 4, 2)]
     plan = launches(plan_lib, 1024, 32768, 1024)
@@ -136,3 +137,37 @@ def test_every_exact_mfma_kind_is_chosen(plan_lib):
     count = C.c_uint32()
     seen = plan_lib.lin_exact_kinds(C.byref(count))
     assert seen == (1 << count.value) - 1, bin(seen)
+
+
+def test_gpu_test_shapes_take_the_kernels_they_name(plan_lib):
+    """The shapes of test_gpu_linear.py that stand for one kernel take it, so
+    that a later rule cannot leave a kernel untested; and between them the EXACT
+    f32-MFMA shapes launch every kind, each with more groups than wavefronts and
+    a ragged last round."""
+    import test_gpu_linear as t
+
+    gemm, fast, mfma, tile = 1, 2, 4, 5  # LinRoute
+
+    def route(mode_fast, m, n, k, f32=False):
+        return plan_lib.lin_route_of(mode_fast, m, n, k, f32, 1)
+
+    assert [route(1, *s) for s in t.FAST_PROMPT] == [gemm] * len(t.FAST_PROMPT)
+    assert [route(1, *s) for s in t.FAST_LAUNCHES] == [fast] * len(t.FAST_LAUNCHES)
+    assert all(len(check(plan_lib, m, n, k)) == 2 for m, n, k, _ in t.FAST_LAUNCHES)
+    assert [route(0, *s) for s in t.EXACT_TILE_CHUNKS] == [tile] * len(t.EXACT_TILE_CHUNKS)
+    m, n, k, f32 = t.EXACT_TILE_CHUNKS[0]
+    assert f32 and (32 << 20) // (k // 128 * n * 4) < m  # more than one launch
+    assert [route(0, *s) for s in t.EXACT_MFMA] == [mfma] * len(t.EXACT_MFMA)
+    several, two = set(), 0
+    a, b = C.c_uint32(), C.c_uint32()
+    for m, n, k in t.EXACT_MFMA:
+        groups = k // 128
+        first = plan_lib.lin_exact(C.c_uint32(m), C.c_uint32(n), C.c_uint32(groups), C.byref(a), C.byref(b))
+        two += first < m
+        plan_lib.lin_exact(C.c_uint32(first), C.c_uint32(n), C.c_uint32(groups), C.byref(a), C.byref(b))
+        if groups > b.value and groups % b.value and n % 64:
+            several.add((a.value, b.value))
+    assert several == {(4, 4), (4, 16), (8, 4), (16, 4), (16, 8), (32, 4)} and two, several
+    # the upper-scale test: the MFMA and the single-token kernel, and the tiles with f32 scales
+    assert route(0, 5, 200, 1024) == mfma and route(0, 1, 200, 1024) == 3
+    assert route(0, 5, 200, 1024, True) == tile
