@@ -136,9 +136,10 @@ __device__ __forceinline__ uint32_t requant_code_bits(uint32_t amax) {
 // up to 2^100 by the hardware's conversion (round to nearest even; the scale
 // keeps every value within 448, where both gave the same code for every f32),
 // past it and for a NaN, whose code differs, by the bitwise one.
-// The bitwise conversion for all (about 20 instructions a value) took the
-// 512-token prefill 0.9 % longer (now 733 us), the official one of 1,024 tokens
-// 0.8 % (992), act quant [512, 8192] with its projection 62.8 us instead of 60.9.
+// The bitwise conversion for all (about 20 instructions a value), in turn on one
+// card where two runs of a side differ by 0.1 % at most, us: 512-token prefill
+// 734.1 (so 727.8), official prefill of 1,024 tokens 989.8 (983.9), act quant
+// with its projection [512, 8192] 62.5 (60.8) and [1, 1024] 11.1 (10.85).
 struct GroupQuant {
   uint32_t code;
   float inv;

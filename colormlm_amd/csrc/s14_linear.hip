@@ -181,7 +181,8 @@ __global__ __launch_bounds__(256) void k_linear_exact(LinearArgs a) {
 
 // ---------------------------------------------------------------------------
 // EXACT, tiled (k % 128 == 0, 16-byte aligned x and w; f32 scales, whose
-// products are not exact in f32, or few tokens over a long k): one wavefront per
+// products are not exact in f32, few tokens over a long k, or few rows and
+// tokens): one wavefront per
 // (64-row tile, scale group g, block of MT tokens), four independent
 // wavefronts per workgroup.  The wavefront DMA-loads its 64 rows x 128 bytes
 // of weight into LDS (buffer_load ... lds: 8 lanes per row, whole lines per
@@ -642,10 +643,13 @@ __global__ __launch_bounds__(64) void k_linear_fast(LinearArgs a, LinearWorkspac
 // 256 bytes sits at p ^ (token & 15).  Sums of kLgFlush groups (one with f32
 // scales, scaled by sa * sb) are added to the running sums, which keeps the
 // rounding of the 512-k sums that k_linear_fast's splits make.  K splits
-// (of 512 k at least) leave their sums in the workspace for k_linear_sum.
-// Bound by the decoding, the MFMAs and the LDS reads in turn: 54 us for 512
-// tokens of wo_a, where the MFMAs alone take 20 (k_linear_fast, one wavefront
-// per 32 x 32 tile and split, 557).  Measured and not kept: 128 tokens a
+// (of 512 k, the last one of what is left) leave their sums in the workspace
+// for k_linear_sum.
+// Bound by the LDS, the MFMAs and the decoding in turn: of the 49 us of 512
+// tokens of wo_a or wo_b (counters, 2.3 GHz) the LDS is busy for 22, half of
+// them bank conflicts, the MFMAs take 14 and the other vector instructions 13
+// or more (the converters run at half rate); k_linear_fast, one wavefront per
+// 32 x 32 tile and split, took 557.  Measured and not kept: 128 tokens a
 // workgroup (one workgroup per CU by registers: 58), every group's sums
 // joined on their own (85), scheduling groups that place the decoding between
 // the MFMAs by hand (61 to 68).
@@ -1032,8 +1036,10 @@ __global__ __launch_bounds__(64 * kGxWaves) void k_linear_gemv_exact(LinearArgs 
 // partial goes to memory.  A group's weights (8 KiB) and its tokens' codes
 // come by coalesced DMA loads into LDS, from where the lane that feeds a row
 // takes its 128 bytes to registers; the next group's loads are in flight
-// during the products.  (Loaded straight to registers, 64 rows' 16 bytes an
-// instruction, the loads' addresses bound the kernel.)  Lane l feeds row l
+// during the products (with 8 tokens the compiler waits for them first: it
+// moves the scale codes, the last loads issued, to other registers).  (Loaded
+// straight to registers, 64 rows' 16 bytes an instruction, the loads'
+// addresses bound the kernel.)  Lane l feeds row l
 // and token l % kT; a lane's result quads: kT = 32 (v_mfma_f32_32x32x1_2b)
 // rows 8 q + 4 (l / 32) + j, kT = 16 (16x16x1_4b) rows 16 q + 4 (l / 16) + j,
 // kT = 4 (4x4x1_16b) rows 4 (l / 4) + j.
@@ -1107,7 +1113,7 @@ __global__ __launch_bounds__(64 * W) void k_linear_exact_mfma(LinearArgs a, uint
       for (uint32_t j = 0; j < kTok / 8u; ++j)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lt_lds_void *)(xm_x[wave] + 1024u * j), 16,
                                                  min(m0 + 8u * j + drow, M - 1u) * K + g * kLinGroup + dpiece, 0, 0, 0);
-    } else {  // four tokens: the lanes past them repeat the last one's line into an unused part
+    } else {  // four tokens: the lanes past their 512 bytes are off (the next wavefront's codes follow)
       if (lane < 8u * kTok)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lt_lds_void *)(xm_x[wave]), 16,
                                                  min(m0 + drow, M - 1u) * K + g * kLinGroup + dpiece, 0, 0, 0);

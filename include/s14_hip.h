@@ -354,12 +354,13 @@ int s14_last_prefill_stats(s14_ctx *ctx, uint32_t *distinct, uint32_t *max_token
  *     activations;
  *   ht, hts: the SwiGLU output of each (token, expert) pair, requantised
  *     the same way, in work-item tiles: item i's tile is 65536 bytes at
- *     ht + 65536 i, byte (s, part, lane, b) at 2048 s + 1024 part +
- *     16 lane + b holding the code of h value 64 s + 32 (lane / 32) +
- *     16 part + b of the pair first_i + (lane % 32); its scales are 2048
- *     bytes at hts + 2048 i, u32 [s / 4][lane] with byte s % 4 = the E8M0
- *     of h values 64 s + 32 (lane / 32) .. +31;
- *   down [n_pairs][4096] f32: each pair's w2 output, route weight not applied;
+ *     ht + 65536 i, byte 4096 u + 2048 (c / 16) + 1024 p + 256 b +
+ *     16 (c % 16) + e holding the code of h value 128 u + 32 b + 16 p + e of
+ *     the pair first_i + c; its scales are 4096 bytes at hts + 4096 i, byte
+ *     512 (u / 2) + 256 (c / 16) + 64 b + 4 (c % 16) + u % 2 = the E8M0 of h
+ *     values 128 u + 32 b .. +31;
+ *   down [n_pairs][4096] f32: each pair's w2 output, route weight not applied
+ *     (official mode: bf16 values, the weight on h);
  *   pair_token [n_pairs]: the token of each pair; token_pair [tokens][7]:
  *     each token's pairs in route order, the shared expert's last;
  *   items [n_items][3]: {expert, first pair, pairs} of each GEMM work item.
